@@ -309,30 +309,99 @@ __global__ __launch_bounds__(64 * kW8Waves, 1) void head_w8_mfma_kernel(
 }
 
 // Per-row argmax of bf16 logits [M, N] (row stride ld): the first NaN if any,
-// else the first maximum (torch.argmax / numpy).  One block per row; every
-// thread scans a strided slice, keys are order-preserving images of the value
-// over the complemented column, so the unsigned maximum is the answer.
-__global__ __launch_bounds__(256) void logits_argmax_kernel(const uint16_t* __restrict__ logits, int N, int64_t ld,
-                                                            int64_t* __restrict__ argmax) {
-    __shared__ uint64_t s_best[256];
-    const int row = blockIdx.x, tid = threadIdx.x;
+// else the first maximum (torch.argmax / numpy).  Keys are order-preserving
+// images of the value over the complemented column, so the unsigned maximum is
+// the answer.
+//
+// A row is cut into parts of kArgPart columns, one block each; a thread loads
+// kArgLoads 16-byte pieces before it looks at any of them (a wave reads 1 KB
+// contiguous per load).  Bound by the round trip of those loads: one block per
+// row with 2-byte loads, one at a time, took ~265 us at N = 248320 for 1 row
+// as for 32, three times the head before it; a whole row in one wide block is
+// still ~7 us of key arithmetic on one CU.  With more than one part, the
+// blocks meet in argmax[row] itself (cleared by the launch before): one
+// 64-bit atomic maximum per block, and logits_argmax_finish turns the winning
+// key into its column.  W8 head and hand-off at N = 248320, 1 row 341 -> 98 us,
+// 32 rows 400 -> 126 us.  Tokens that live in host memory, where device atomics
+// do not reach, keep one block per row, which walks the parts (11 us alone).
+constexpr int kArgThreads = 512, kArgLoads = 4, kArgPart = kArgThreads * 8 * kArgLoads;
+
+__device__ __forceinline__ uint64_t argmax_key(uint32_t b, int c) {
+    const bool nan = (b & 0x7fffu) > 0x7f80u;
+    const uint32_t mag = (b & 0x8000u) ? ((b & 0x7fffu) ? (~b & 0xffffu) : 0x8000u) : (b | 0x8000u);
+    const uint32_t ord = nan ? 0x1ffffu : mag;            // every NaN above +inf
+    return (uint64_t(ord) << 32) | uint32_t(~c);
+}
+
+template <bool SPLIT>
+__global__ __launch_bounds__(kArgThreads) void logits_argmax_kernel(const uint16_t* __restrict__ logits, int N,
+                                                                    int64_t ld, int64_t* __restrict__ argmax) {
+    __shared__ uint64_t s_best[kArgThreads / 64];
+    const int row = blockIdx.y, tid = threadIdx.x;
     const uint16_t* src = logits + size_t(row) * size_t(ld);
+    // 16-byte pieces on the address grid: piece p is columns 8 p - lead .. 8 p - lead + 7
+    // (lead columns of the first piece, and those past N, are not the row's)
+    const int lead = int((reinterpret_cast<uintptr_t>(src) >> 1) & 7);
     uint64_t best = 0;
-    for (int c = tid; c < N; c += 256) {
-        const uint32_t b = src[c];
-        const bool nan = (b & 0x7fffu) > 0x7f80u;
-        const uint32_t mag = (b & 0x8000u) ? ((b & 0x7fffu) ? (~b & 0xffffu) : 0x8000u) : (b | 0x8000u);
-        const uint32_t ord = nan ? 0x1ffffu : mag;        // every NaN above +inf
-        const uint64_t key = (uint64_t(ord) << 32) | uint32_t(~c);
+    auto take = [&](uint32_t b, int c) {
+        const uint64_t key = argmax_key(b, c);
         best = key > best ? key : best;
+    };
+    for (int64_t base = int64_t(blockIdx.x) * kArgPart - lead; base < N; base += int64_t(gridDim.x) * kArgPart) {
+        u32x4 v[kArgLoads];
+        bool whole[kArgLoads];
+#pragma unroll
+        for (int u = 0; u < kArgLoads; ++u) {
+            const int64_t c = base + 8 * (int64_t(u) * kArgThreads + tid);
+            whole[u] = c >= 0 && c + 8 <= N;
+            if (whole[u]) v[u] = *reinterpret_cast<const u32x4*>(src + c);
+        }
+#pragma unroll
+        for (int u = 0; u < kArgLoads; ++u) {
+            const int64_t c = base + 8 * (int64_t(u) * kArgThreads + tid);
+            if (whole[u]) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    take(v[u][e] & 0xffffu, int(c) + 2 * e);
+                    take(v[u][e] >> 16, int(c) + 2 * e + 1);
+                }
+            } else {
+                for (int64_t k = c < 0 ? 0 : c; k < c + 8 && k < N; ++k) take(src[k], int(k));
+            }
+        }
     }
-    s_best[tid] = best;
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+        const uint64_t o = __shfl_xor(best, m, 64);
+        best = o > best ? o : best;
+    }
+    if ((tid & 63) == 0) s_best[tid >> 6] = best;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (tid < s) s_best[tid] = s_best[tid] > s_best[tid + s] ? s_best[tid] : s_best[tid + s];
-        __syncthreads();
+    if (tid != 0) return;
+#pragma unroll
+    for (int w = 1; w < kArgThreads / 64; ++w) best = s_best[w] > best ? s_best[w] : best;
+    if constexpr (SPLIT) {
+        // (a part past the row's last column, when the lead makes one more, holds no key)
+        if (best) atomicMax(reinterpret_cast<unsigned long long*>(argmax + row), (unsigned long long)best);
+    } else {
+        argmax[row] = int64_t(~uint32_t(best));
     }
-    if (tid == 0) argmax[row] = int64_t(~uint32_t(s_best[0]));
+}
+
+// argmax[row]: winning key -> its column
+__global__ __launch_bounds__(64) void logits_argmax_finish_kernel(int M, int64_t* __restrict__ argmax) {
+    const int row = blockIdx.x * 64 + threadIdx.x;
+    if (row < M) argmax[row] = int64_t(~uint32_t(uint64_t(argmax[row])));
+}
+
+// Memory of a device (hipMalloc), as opposed to pinned host or managed memory.
+bool device_memory(const void* p) {
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && !at.isManaged;
 }
 
 bool head_shape(int N) { return N == 256 || N == 1024 || N == 4096 || N == 65536 || N == 248320; }
@@ -428,7 +497,25 @@ extern "C" hipError_t ornith_logits_argmax_launch(const void* logits_bf16, int M
     const Buffer buffers[] = {{logits_bf16, (size_t(M - 1) * size_t(ld) + size_t(N)) * 2, 2, false, false},
                               {argmax_i64, size_t(M) * 8, 8, true, false}};
     if (!check_buffers(buffers)) return hipErrorInvalidValue;
-    timed_launch("logits_argmax", logits_argmax_kernel, dim3(M), dim3(256), 0, stream,
-                 static_cast<const uint16_t*>(logits_bf16), N, ld, static_cast<int64_t*>(argmax_i64));
+    // up to 7 columns of lead in the first 16-byte piece
+    const int parts = int((int64_t(N) + 7 + kArgPart - 1) / kArgPart);
+    const auto src = static_cast<const uint16_t*>(logits_bf16);
+    const auto dst = static_cast<int64_t*>(argmax_i64);
+    auto go = [&](auto kernel, int parts) {
+        // rows ride on the grid's y axis (65535 blocks at most)
+        for (int r = 0; r < M; r += 65535)
+            timed_launch("logits_argmax", kernel, dim3(parts, std::min(M - r, 65535)), dim3(kArgThreads), 0, stream,
+                         src + size_t(r) * size_t(ld), N, ld, dst + r);
+    };
+    if (parts == 1 || !device_memory(dst)) {
+        go(logits_argmax_kernel<false>, 1);
+        return hipGetLastError();
+    }
+    hipError_t st = launch_fill_u32(reinterpret_cast<uint32_t*>(dst), size_t(M) * 2, 0u, stream);
+    if (st != hipSuccess) return st;
+    go(logits_argmax_kernel<true>, parts);
+    st = hipGetLastError();
+    if (st != hipSuccess) return st;
+    timed_launch("logits_argmax_finish", logits_argmax_finish_kernel, dim3((M + 63) / 64), dim3(64), 0, stream, M, dst);
     return hipGetLastError();
 }
