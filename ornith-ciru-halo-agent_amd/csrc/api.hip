@@ -213,7 +213,7 @@ hipError_t dense_run(const void* input, const void* codes, const void* meta, voi
     auto sc = at<uint16_t>(ws, l.scales);
     auto su = at<int32_t>(ws, l.sums);
     ProjArgs a{};
-    if (M <= kDenseFusedRows) {
+    if (M <= dense_fused_rows(K)) {
         // the projection prepares its own activations
         a.dense_x = static_cast<const uint16_t*>(input);
         a.flag_input = kDenseNonfiniteInput;

@@ -127,13 +127,18 @@ struct ProjArgs {
     int N, K, tile;           // tile: 16 or 32 (bank layout)
     uint32_t* sticky;
     uint32_t flag_projection, flag_bf16;
-    // dense, rows <= kDenseFusedRows: bf16 input [rows, K]; the projection
+    // dense, rows <= dense_fused_rows(K): bf16 input [rows, K]; the projection
     // kernel then prepares the activations itself (act_words unused)
     const uint16_t* dense_x;
     uint32_t flag_input, flag_act;
 };
 constexpr int kDenseStreamRows = 64;   // weight-streaming projection up to this many rows
-constexpr int kDenseFusedRows = 8;     // ... with activations prepared in the same kernel
+// ... with the activations prepared in the same kernel up to this many rows.
+// Every block repeats that work, four rows per pass and one wave per 256-group:
+// one pass costs less than the launch it saves at every K (4 rows, K = 2048:
+// 5.3 against ~7 us), two only where a block has few groups (8 rows, fused
+// against separate: K = 512 4.7 / 6.0 us, K = 2048 7.2 / 7.3, K = 4096 10.8 / 7.8).
+inline int dense_fused_rows(int K) { return K <= 4 * kGroup ? 8 : 4; }
 hipError_t launch_project_gemv(const ProjArgs& a, int max_segments, Out mode, hipStream_t s);
 
 // Grouped int8-MFMA projection over the permuted routes (prefill path).

@@ -138,201 +138,255 @@ __global__ __launch_bounds__(256) void project_gemv_kernel(ProjArgs a, int NT, i
     }
 }
 
-// Dense weight-streaming projection for up to kStreamRows rows (decode and
-// small batches).  One block of 4 waves owns COLS (32, or 16 on tile-16
-// banks above kDenseNarrowRows rows) consecutive output columns;
-// half-wave h of the block owns group g0 + h of the current 8-group pass.
-// Each lane keeps its 32 code words of that group in registers (every load of
-// the block is issued before the first dot), so one pass over the bank moves
-// the whole weight through HBM once however many rows there are.
-//   tile 32: lane L holds column L, words j*32 + L of block (tile, g).
-//   tile 16: lane L = 16*jp + n holds words (2i+jp)*16 + n (i < 16) of the two
-//            16-column blocks of the 32-column unit; the two half-dots of a
-//            column meet across lanes L and L^16, after which lane L keeps
-//            column L of the unit.  With 16 columns a lane holds the words
-//            of its one block and lanes L, L^16 both end with column n.
-// FUSED (a.dense_x set, up to kDenseFusedRows rows): the block also prepares
-// its activations from the bf16 input: the H128 +
-// group-256 int8 recipe of act_bf16_block, 16 lanes per (row, group), written
-// to LDS instead of the workspace.  Every block repeats this small amount of
-// work; the first chunk's inputs are loaded before the code words, so it runs
-// while the weights are in flight and the separate activation launch goes.
-// Otherwise the activations come from the workspace (act_words/scales/sums).
-// Terms go through LDS; one thread per (row, column) adds them in group order
-// (the fp32 tree of dense_g256_consumer.cpp:116-143), so results equal
-// project_gemv_kernel's bit for bit.
-constexpr int kStreamRows = kDenseStreamRows;   // rows whose running sums stay in LDS
-constexpr int kStreamChunk = 8;     // rows per term pass (8 rows x 32 columns = 256 threads)
-// Tile-16 banks above this many rows (the activations read from the
-// workspace) run 16-column blocks: twice the blocks, each lane streaming one
-// 16-column tile.  One-row-per-block latency favours 32 columns below it
-// (graph-timed per call, 16 against 32 columns: 1 row 6.0 / 5.55 us, 8 rows
-// 15.8 / 12.6, 16 rows 15.8 / 16.1, 32 rows 24.5 / 25.6, 64 rows 40.9 / 44.1).
-constexpr int kDenseNarrowRows = 16;
+// Dense weight-streaming projection for up to kDenseStreamRows rows on the
+// int8 matrix cores.  One block owns 32 output columns; wave w owns 256-group
+// w of the current NW-group pass, so every load of the block is issued before
+// its first product and the bank crosses HBM once for any row count.
+//  - Codes: load u (0..7) of lane li + 16q takes word j = 4u + q of column li
+//    of each 16-column half, so a load of an N16 tile is 256 contiguous bytes
+//    (of an N32 tile four 64-byte halves of its rows; the other half's load
+//    takes the rest).  v_mfma_i32_16x16x64_i8 s pairs words u = 2s, 2s + 1
+//    (unpacked: even codes, odd codes) with activation chunks 8s + q and
+//    8s + 4 + q.  Any pairing of K is exact: |dot| < 2^19.
+//  - The product is (codes x activations): lane li + 16q ends with columns
+//    4q + 0..3 of activation row li, so a row's scale and sum are one value
+//    per lane and the four columns' metadata one 16-byte load.
+//  - Terms (tree_term) meet in LDS; one thread per (row, column) adds them in
+//    ascending group order (the fp32 tree of dense_g256_consumer.cpp:116-143),
+//    so results equal project_gemv_kernel's bit for bit.
+// FP > 0 (a.dense_x set): the wave also prepares its group of the activations
+// from the bf16 input, FP passes of four rows (the recipe of act_bf16_block),
+// into LDS while its codes are in flight; every block repeats that work, so it
+// is done up to dense_fused_rows rows, and above them the activations come from
+// the workspace.
+// Bound by latency: the weights of a 6144 x 2048 linear are 1 us of HBM time;
+// a call is the kernel boundaries (~1.1 us each), the loads' round trip and the
+// two exchanges through LDS.  Graph-timed per call at 6144 x 2048, activation
+// launch included, against the v_dot4 kernel before it (rows one after another
+// on the VALU): 1 row 5.4 -> 5.0 us, 4 rows 8.0 -> 5.3, 8 rows 12.3 -> 7.2,
+// 16 rows 15.7 -> 7.6, 32 rows 23.5 -> 9.4, 64 rows 39.5 -> 12.1; at 2048 x
+// 4096 1 row 8.0 -> 6.3, 32 rows 37.8 -> 10.8, 64 rows 69.2 -> 17.7.
+typedef int mfma_i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));   // metadata is 4-byte aligned
 
-template <int TILE, bool FUSED, int COLS = 32>
-__global__ __launch_bounds__(256) void dense_stream_kernel(ProjArgs a) {
-    static_assert(COLS == 32 || TILE == 16, "16-column blocks read the N16 layout");
-    __shared__ uint32_t la[kStreamChunk][8 * 64];
-    __shared__ float lsa[kStreamChunk][8], lss[kStreamChunk][8];
-    __shared__ float lterm[kStreamChunk][8][32];
-    __shared__ float lrun[kStreamRows][32];
+template <int TILE, int MT, int FP, int NW>
+__global__ __launch_bounds__(64 * NW) void dense_stream_kernel(ProjArgs a) {
+    static_assert(FP == 0 || (MT == 1 && FP <= 2), "fused rows fit one row tile");
+    constexpr int ROWS = 16 * MT, NT = 64 * NW, OUT = (ROWS * 32 + NT - 1) / NT;
+    constexpr int kTermStride = 36;                // floats per row: 16-byte stores spread over the banks
+    constexpr int kActStride = 72;                 // words per row: conflict-free 8-byte reads
+    // one LDS area per wave: its activation rows (32 at a time), then its terms
+    constexpr int kActRows = ROWS < 32 ? ROWS : 32;
+    constexpr int kWaveWords = kActRows * kActStride > ROWS * kTermStride ? kActRows * kActStride : ROWS * kTermStride;
+    __shared__ __attribute__((aligned(16))) uint32_t s_wave[NW][kWaveWords];
+    __shared__ float2 s_scale[FP ? NW : 1][FP ? 16 : 1];
 
-    const int tid = threadIdx.x, hw = tid >> 5, L = tid & 31, jp = L >> 4, n16 = L & 15;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, q = lane >> 4;
     const int GS = a.K / kGroup, M = a.dense_rows;
-    const int col0 = blockIdx.x * COLS, col = col0 + (COLS == 16 ? n16 : L);
-    for (int g0 = 0; g0 < GS; g0 += 8) {
-        const int g = g0 + hw, gc = min(8, GS - g0);
-        const bool gv = g < GS;
-        // Loads are unconditional (a predicated load would drain the queue):
-        // a half-wave past the last group reads group GS-1 and writes no term;
-        // a missing second 16-column block reads the first one, whose dots
-        // only reach columns >= N, which are never written.
-        const int gq = gv ? g : GS - 1;
-        // input words of the first chunk's first pair pass (fused activations)
-        auto xsrc = [&](int r0, int nr, int p0) {
-            const int pc = min(p0 + (tid >> 4), nr * gc - 1);
-            return a.dense_x + size_t(r0 + pc / gc) * a.K + (g0 + pc % gc) * kGroup + quarter_base(tid & 15);
-        };
-        uint4 px0 = make_uint4(0, 0, 0, 0), px1 = px0;
-        if constexpr (FUSED) {
-            const uint16_t* xp0 = xsrc(0, min(kStreamChunk, M), 0);
-            px0 = *reinterpret_cast<const uint4*>(xp0);
-            px1 = *reinterpret_cast<const uint4*>(xp0 + 8);
-        }
-        uint32_t wr[32];
-        uint32_t mw;
-        if (TILE == 32) {
-            const uint32_t* wp = a.codes + (size_t(blockIdx.x) * GS + gq) * 1024 + L;
+    // a missing second 16-column half (N % 32 == 16) repeats the first; its
+    // columns are never written
+    const int half1 = 2 * int(blockIdx.x) + 1 < (a.N >> 4) ? 1 : 0;
+    float run[OUT];
 #pragma unroll
-            for (int j = 0; j < 32; ++j) wr[j] = load_once(wp + j * 32);
-            mw = a.meta[(size_t(blockIdx.x) * GS + gq) * 32 + L];
+    for (int i = 0; i < OUT; ++i) run[i] = 0.f;
+    uint32_t flags = 0;
+    uint32_t* s_act = s_wave[w];
+    // the wave's own LDS words, written by other lanes of it
+    auto wave_fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+
+    for (int g0 = 0; g0 < GS; g0 += NW) {
+        // a wave past the last group reads group GS - 1 and writes no term
+        const int g = min(g0 + w, GS - 1);
+        const bool gv = g0 + w < GS;
+        // ---- inputs (fused), then codes and metadata, then the workspace's activations ----
+        uint4 xa[FP ? FP : 1][2];
+        if constexpr (FP > 0) {
+#pragma unroll
+            for (int i = 0; i < FP; ++i) {
+                const uint16_t* src = a.dense_x + size_t(min(4 * i + q, M - 1)) * a.K + g * kGroup + quarter_base(li);
+                xa[i][0] = *reinterpret_cast<const uint4*>(src);
+                xa[i][1] = *reinterpret_cast<const uint4*>(src + 8);
+            }
+        }
+        uint32_t wr[2][8];
+        u32x4 mw[2];
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) {
+            const uint32_t* src;
+            const uint32_t* msrc;
+            if constexpr (TILE == 32) {
+                src = a.codes + (size_t(blockIdx.x) * GS + g) * 1024 + 32 * q + 16 * ct + li;
+                msrc = a.meta + (size_t(blockIdx.x) * GS + g) * 32 + 16 * ct + 4 * q;
+            } else {
+                const size_t block = size_t(2 * int(blockIdx.x) + (ct ? half1 : 0)) * GS + g;
+                src = a.codes + block * 512 + 16 * q + li;
+                msrc = a.meta + block * 16 + 4 * q;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) wr[ct][u] = load_once(src + u * 4 * TILE);
+            mw[ct] = *reinterpret_cast<const u32x4_a4*>(msrc);
+        }
+        uint2 fa2[MT][8];                          // [row tile][2s + e]: chunk 8s + 4e + q
+        float sa[MT], ss[MT];
+        if constexpr (FP == 0) {
+            // 16 lanes per row, four rows per load; each half of 32 rows
+            // passes through LDS into the products' layout (loaded straight
+            // in it, 32 bytes of 16 rows per instruction, the call took 17.1
+            // instead of 12.1 us at 64 rows, 11.9 instead of 9.4 at 32)
+            u32x4 av[ROWS / 4];
+#pragma unroll
+            for (int i = 0; i < ROWS / 4; ++i)
+                av[i] = *reinterpret_cast<const u32x4*>(a.act_words + size_t(min(4 * i + q, M - 1)) * (a.K / 4) +
+                                                        g * 64 + 4 * li);
+            uint32_t sbits[MT];
+            int sum[MT];
+#pragma unroll
+            for (int rt = 0; rt < MT; ++rt) {
+                const int row = min(16 * rt + li, M - 1);
+                sbits[rt] = a.act_scales[size_t(row) * GS + g];
+                sum[rt] = a.act_sums[size_t(row) * GS + g];
+            }
+#pragma unroll
+            for (int h = 0; h < ROWS / kActRows; ++h) {
+                if (h) wave_fence();
+#pragma unroll
+                for (int i = 0; i < kActRows / 4; ++i)
+                    *reinterpret_cast<u32x4*>(&s_act[(4 * i + q) * kActStride + 4 * li]) = av[h * (kActRows / 4) + i];
+                wave_fence();
+#pragma unroll
+                for (int rt = 0; rt < kActRows / 16; ++rt)
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        fa2[h * (kActRows / 16) + rt][u] =
+                            *reinterpret_cast<const uint2*>(&s_act[(16 * rt + li) * kActStride + 8 * u + 2 * q]);
+            }
+#pragma unroll
+            for (int rt = 0; rt < MT; ++rt) {
+                sa[rt] = f16_bits_to_f32(uint16_t(sbits[rt]));
+                ss[rt] = sa[rt] * float(sum[rt]);
+            }
         } else {
-            const int tA = COLS == 16 ? int(blockIdx.x) : 2 * int(blockIdx.x);
-            const int tB = (tA + 1) * 16 < a.N ? tA + 1 : tA;
-            const uint32_t* pa = a.codes + (size_t(tA) * GS + gq) * 512 + jp * 16 + n16;
-            const uint32_t* pb = a.codes + (size_t(tB) * GS + gq) * 512 + jp * 16 + n16;
+            // the input's first use stays behind the code loads (its wait
+            // would otherwise come before they are issued)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                wr[i] = load_once(pa + i * 32);
-                if (COLS == 32) wr[16 + i] = load_once(pb + i * 32);
-            }
-            const int cq = min(col, a.N - 1);
-            mw = a.meta[(size_t(cq >> 4) * GS + gq) * 16 + (cq & 15)];
-        }
-        // the input's first use stays behind the weight loads (its wait would
-        // otherwise come before they are issued)
-        asm volatile("" : "+v"(px0.x), "+v"(px0.y), "+v"(px0.z), "+v"(px0.w), "+v"(px1.x), "+v"(px1.y), "+v"(px1.z),
-                     "+v"(px1.w));
-        for (int r0 = 0; r0 < M; r0 += kStreamChunk) {
-            const int nr = min(kStreamChunk, M - r0);
-            __syncthreads();
-            // ---- this chunk's activation words, scales and scaled sums ----
-            if constexpr (!FUSED) {
-                for (int q = tid; q < nr * gc * 16; q += 256) {
-                    const int r = q / (gc * 16), w4 = q % (gc * 16);
-                    *reinterpret_cast<uint4*>(&la[r][w4 * 4]) = *reinterpret_cast<const uint4*>(
-                        a.act_words + size_t(r0 + r) * (a.K / 4) + size_t(g0) * 64 + w4 * 4);
-                }
-                if (tid < nr * gc) {
-                    const int r = tid / gc, gl = tid % gc;
-                    const float sa = f16_bits_to_f32(a.act_scales[size_t(r0 + r) * GS + g0 + gl]);
-                    lsa[r][gl] = sa;
-                    lss[r][gl] = sa * float(a.act_sums[size_t(r0 + r) * GS + g0 + gl]);
-                }
-            }
-            const int pairs = FUSED ? nr * gc : 0, l = tid & 15;
-            for (int p0 = 0; p0 < pairs; p0 += 16) {
-                uint4 x0 = px0, x1 = px1;
-                if (r0 != 0 || p0 != 0) {
-                    const uint16_t* xp = xsrc(r0, nr, p0);
-                    x0 = *reinterpret_cast<const uint4*>(xp);
-                    x1 = *reinterpret_cast<const uint4*>(xp + 8);
-                }
-                const uint32_t u[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            for (int i = 0; i < FP; ++i)
+                asm volatile("" : "+v"(xa[i][0].x), "+v"(xa[i][0].y), "+v"(xa[i][0].z), "+v"(xa[i][0].w),
+                                  "+v"(xa[i][1].x), "+v"(xa[i][1].y), "+v"(xa[i][1].z), "+v"(xa[i][1].w));
+#pragma unroll
+            for (int i = 0; i < FP; ++i) {
+                const uint32_t u[8] = {xa[i][0].x, xa[i][0].y, xa[i][0].z, xa[i][0].w,
+                                       xa[i][1].x, xa[i][1].y, xa[i][1].z, xa[i][1].w};
                 float v[16];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     v[2 * e] = bf16_bits_to_f32(u[e] & 0xffffu);
                     v[2 * e + 1] = bf16_bits_to_f32(u[e] >> 16);
                 }
-                uint32_t flags = 0;
+                uint32_t f = 0;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) if (!isfinite(v[e])) flags |= a.flag_input;
+                for (int e = 0; e < 16; ++e) if (!isfinite(v[e])) f |= a.flag_input;
                 h128_quarter(v);
                 uint32_t w4[4];
                 uint16_t sbits;
                 int sum;
-                quantize_quarter_fast<127>(v, w4, sbits, sum, flags, a.flag_input | a.flag_act, a.flag_act);
-                const int pi = p0 + (tid >> 4);
-                if (pi < pairs) {
-                    const int r = pi / gc, gl = pi % gc;
-                    *reinterpret_cast<uint4*>(&la[r][gl * 64 + quarter_base(l) / 4]) =
-                        make_uint4(w4[0], w4[1], w4[2], w4[3]);
-                    if (l == 0) {
-                        const float sa = f16_bits_to_f32(sbits);
-                        lsa[r][gl] = sa;
-                        lss[r][gl] = sa * float(sum);
-                    }
-                    flag_or(a.sticky, flags);
+                quantize_quarter_fast<127>(v, w4, sbits, sum, f, a.flag_input | a.flag_act, a.flag_act);
+                const int row = 4 * i + q;         // rows past M repeat row M - 1
+                *reinterpret_cast<uint4*>(&s_act[row * kActStride + quarter_base(li) / 4]) =
+                    make_uint4(w4[0], w4[1], w4[2], w4[3]);
+                if (li == 0) {
+                    const float scale = f16_bits_to_f32(sbits);
+                    s_scale[w][row] = make_float2(scale, scale * float(sum));
+                }
+                flags |= f;
+            }
+            wave_fence();
+            const int row = min(li, min(4 * FP, M) - 1);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                fa2[0][u] = *reinterpret_cast<const uint2*>(&s_act[row * kActStride + 8 * u + 2 * q]);
+            const float2 sc = s_scale[w][row];
+            sa[0] = sc.x;
+            ss[0] = sc.y;
+        }
+        wave_fence();                              // the terms take the activations' place
+        // ---- exact dots and the group's terms ----
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) {
+            mfma_i32x4 acc[MT];
+#pragma unroll
+            for (int rt = 0; rt < MT; ++rt) acc[rt] = mfma_i32x4{0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const uint32_t w0 = wr[ct][2 * s], w1 = wr[ct][2 * s + 1];
+                const mfma_i32x4 fb = {code_even(w0), code_odd(w0), code_even(w1), code_odd(w1)};
+#pragma unroll
+                for (int rt = 0; rt < MT; ++rt) {
+                    const mfma_i32x4 fa = {int(fa2[rt][2 * s].x), int(fa2[rt][2 * s].y), int(fa2[rt][2 * s + 1].x),
+                                           int(fa2[rt][2 * s + 1].y)};
+                    acc[rt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb, fa, acc[rt], 0, 0, 0);
                 }
             }
-            __syncthreads();
-            for (int r = 0; r < nr; ++r) {
-                const uint32_t* ab = &la[r][hw * 64];
-                int dot;
-                if (TILE == 32) {
-                    int d = 0;
+            if (gv) {
 #pragma unroll
-                    for (int c4 = 0; c4 < 16; ++c4) {
-                        const uint4 av = reinterpret_cast<const uint4*>(ab)[c4];
-                        d = dot4(code_even(wr[2 * c4]), int(av.x), d);
-                        d = dot4(code_odd(wr[2 * c4]), int(av.y), d);
-                        d = dot4(code_even(wr[2 * c4 + 1]), int(av.z), d);
-                        d = dot4(code_odd(wr[2 * c4 + 1]), int(av.w), d);
-                    }
-                    dot = d;
-                } else {
-                    int d0 = 0, d1 = 0;
+                for (int rt = 0; rt < MT; ++rt) {
+                    f32x4 t;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const uint2 av = *reinterpret_cast<const uint2*>(&ab[4 * i + 2 * jp]);
-                        d0 = dot4(code_even(wr[i]), int(av.x), d0);
-                        d0 = dot4(code_odd(wr[i]), int(av.y), d0);
-                        if (COLS == 32) {
-                            d1 = dot4(code_even(wr[16 + i]), int(av.x), d1);
-                            d1 = dot4(code_odd(wr[16 + i]), int(av.y), d1);
-                        }
-                    }
-                    const int sA = d0 + xor_perm_i<16>(d0), sB = COLS == 32 ? d1 + xor_perm_i<16>(d1) : sA;
-                    dot = jp ? sB : sA;
+                    for (int r = 0; r < 4; ++r) t[r] = tree_term(acc[rt][r], sa[rt], ss[rt], mw[ct][r]);
+                    *reinterpret_cast<f32x4*>(&s_wave[w][(16 * rt + li) * kTermStride + 16 * ct + 4 * q]) = t;
                 }
-                // 16-column blocks: lanes L and L ^ 16 hold the same column
-                if (gv && (COLS == 32 || jp == 0)) lterm[r][hw][L] = tree_term(dot, lsa[r][hw], lss[r][hw], mw);
-            }
-            __syncthreads();
-            const int r = tid >> 5;
-            if (r < nr && (COLS == 32 || L < 16)) {
-                float v = g0 == 0 ? 0.f : lrun[r0 + r][L];
-                for (int gl = 0; gl < gc; ++gl) v = v + lterm[r][gl][L];
-                lrun[r0 + r][L] = v;
             }
         }
+        __syncthreads();
+        const int gc = min(NW, GS - g0);
+#pragma unroll
+        for (int i = 0; i < OUT; ++i) {
+            const int r = min((tid >> 5) + i * (NT / 32), ROWS - 1), c = tid & 31;
+            for (int gl = 0; gl < gc; ++gl) run[i] = run[i] + __uint_as_float(s_wave[gl][r * kTermStride + c]);
+        }
+        if (g0 + NW < GS) __syncthreads();
     }
-    __syncthreads();
-    for (int q = tid; q < M * COLS; q += 256) {
-        const int r = q / COLS, c = col0 + q % COLS;
-        if (c >= a.N) continue;
-        const float v = lrun[r][q % COLS];
+#pragma unroll
+    for (int i = 0; i < OUT; ++i) {
+        const int r = (tid >> 5) + i * (NT / 32), c = 32 * int(blockIdx.x) + (tid & 31);
+        if (r >= M || c >= a.N) continue;
+        const float v = run[i];
         const size_t o = size_t(r) * a.N + c;
         const uint16_t b = f32_to_bf16_bits(v);
-        uint32_t f = 0;
-        if (!isfinite(v)) f |= a.flag_projection;
-        if ((b & 0x7f80u) == 0x7f80u) f |= a.flag_bf16;
+        if (!isfinite(v)) flags |= a.flag_projection;
+        if ((b & 0x7f80u) == 0x7f80u) flags |= a.flag_bf16;
         if (a.out) a.out[o] = v;
         if (a.out_bf16) a.out_bf16[o] = b;
-        flag_or(a.sticky, f);
     }
+    flag_or(a.sticky, flags);
+}
+
+// Waves per block: one per 256-group of K up to 16 (8 with 64 rows, whose
+// activations take the registers of a 16-wave block), at least 4.
+template <int TILE, int MT, int FP> void go_dense_stream(const ProjArgs& a, hipStream_t s) {
+    const dim3 grid((a.N + 31) / 32);
+    const int GS = a.K / kGroup;
+    if (GS <= 4 || FP > 1)                         // eight fused rows: K <= 1024 (dense_fused_rows)
+        timed_launch("dense_stream", dense_stream_kernel<TILE, MT, FP, 4>, grid, dim3(256), 0, s, a);
+    else if constexpr (FP <= 1) {
+        if (GS <= 8 || MT > 2)
+            timed_launch("dense_stream", dense_stream_kernel<TILE, MT, FP, 8>, grid, dim3(512), 0, s, a);
+        else if constexpr (MT <= 2)
+            timed_launch("dense_stream", dense_stream_kernel<TILE, MT, FP, 16>, grid, dim3(1024), 0, s, a);
+    }
+}
+
+template <int TILE> void launch_dense_stream(const ProjArgs& a, hipStream_t s) {
+    const int M = a.dense_rows;
+    if (a.dense_x && M <= 4) go_dense_stream<TILE, 1, 1>(a, s);
+    else if (a.dense_x) go_dense_stream<TILE, 1, 2>(a, s);
+    else if (M <= 16) go_dense_stream<TILE, 1, 0>(a, s);
+    else if (M <= 32) go_dense_stream<TILE, 2, 0>(a, s);
+    else go_dense_stream<TILE, 4, 0>(a, s);
 }
 
 hipError_t launch_project_gemv(const ProjArgs& a, int max_segments, Out mode, hipStream_t s) {
@@ -342,18 +396,9 @@ hipError_t launch_project_gemv(const ProjArgs& a, int max_segments, Out mode, hi
     const int ntiles = (a.N + 31) / 32;
     const dim3 grid(max_segments, (ntiles + NT - 1) / NT);
     if (max_segments <= 0) return hipSuccess;
-    if (mode == Out::Dense && !a.segments && a.dense_rows <= kStreamRows) {
-        const dim3 g((a.N + 31) / 32);
-        if (a.dense_x) {
-            if (a.tile == 32) timed_launch("dense_stream", dense_stream_kernel<32, true>, g, dim3(256), 0, s, a);
-            else timed_launch("dense_stream", dense_stream_kernel<16, true>, g, dim3(256), 0, s, a);
-        } else {
-            if (a.tile == 32) timed_launch("dense_stream", dense_stream_kernel<32, false>, g, dim3(256), 0, s, a);
-            else if (a.dense_rows > kDenseNarrowRows)
-                timed_launch("dense_stream", dense_stream_kernel<16, false, 16>, dim3((a.N + 15) / 16), dim3(256), 0, s,
-                             a);
-            else timed_launch("dense_stream", dense_stream_kernel<16, false>, g, dim3(256), 0, s, a);
-        }
+    if (mode == Out::Dense && !a.segments && a.dense_rows <= kDenseStreamRows) {
+        if (a.tile == 32) launch_dense_stream<32>(a, s);
+        else launch_dense_stream<16>(a, s);
         return hipGetLastError();
     }
     if (a.tile == 32) {
