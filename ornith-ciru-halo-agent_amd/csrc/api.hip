@@ -54,8 +54,9 @@ RoutedPlan routed_plan(int Tcap, bool shared_slot, bool layer) {
     return p;
 }
 
-// Prefill path (T > 32): permutation into expert segments and 64-route
-// tiles, int8-MFMA grouped projections, middle quantisation, slot reduce.
+// Prefill path (T > 32): permutation into expert segments and 16- or 32-route
+// tiles, int8-MFMA grouped projections (the gate-up quantises its middle rows
+// itself), slot reduce.
 hipError_t run_routed(const RoutedPlan& p, void* ws, const void* input, const float* weights, const int32_t* ids,
                       const void* gate_codes, const void* gate_meta, const void* down_codes, const void* down_meta,
                       const void* sg_codes, const void* sg_meta, const void* sd_codes, const void* sd_meta,
@@ -65,20 +66,27 @@ hipError_t run_routed(const RoutedPlan& p, void* ws, const void* input, const fl
     const bool shared = sg_codes != nullptr;
     const int R = T * kTop, RS = R + (shared ? T : 0);
     const PermuteScratch ps = carve_permute(at<void>(ws, p.permute), Tcap * kTop, shared ? Tcap : 0);
+    // the projections' m-tiles are listed in the (otherwise unused) gate_y rows, 4 KiB a route
+    Segment* work = at<Segment>(ws, p.l.gate_y);
+    const int tile_rows = grouped_tile_rows(T);
     auto gw = at<uint32_t>(ws, p.l.gate_low);
     auto gs = at<uint16_t>(ws, p.l.gate_scales);
     auto gsum = at<int32_t>(ws, p.l.gate_sums);
     // the A8 gate input rides on the bank-scan launch (the A4 one has its own)
     const ActJob act{static_cast<const uint16_t*>(input), T, shared ? nullptr : ids, gw, gs, gsum};
-    TRY(launch_permute(ids, R, T, shared, ps, sticky, 64, s, counted, qmax == 127 ? &act : nullptr));
+    TRY(launch_permute(ids, R, T, shared, ps, sticky, work, tile_rows, s, counted, qmax == 127 ? &act : nullptr));
     if (qmax != 127)
         TRY(launch_act_bf16(static_cast<const uint16_t*>(input), kHidden, T, kHidden, qmax, shared ? nullptr : ids, gw,
                             gs, gsum, sticky, kFlagNonfiniteInput, kFlagInvalidActivation, s));
-    const int max_tiles = (RS + 63) / 64 + (R < kExperts ? R : kExperts) + (shared ? 1 : 0);
+    const int max_tiles =
+        (RS + tile_rows - 1) / tile_rows + (R < kExperts ? R : kExperts) + (shared ? 1 : 0);
+    auto dw = at<uint32_t>(ws, p.l.down_low);
+    auto dsc = at<uint16_t>(ws, p.l.down_scales);
+    auto dsum = at<int32_t>(ws, p.l.down_sums);
     MfmaArgs a{};
     a.segments = ps.segments;
-    a.tiles = ps.tiles;
-    a.ntiles = ps.meta + 1;
+    a.tiles = work;
+    a.ntiles = ps.meta + 2;
     a.routes = ps.routes;
     a.R = R;
     a.codes = static_cast<const uint32_t*>(gate_codes);
@@ -89,18 +97,10 @@ hipError_t run_routed(const RoutedPlan& p, void* ws, const void* input, const fl
     a.bank_meta_words = kGateBankMeta;
     a.act_words = gw; a.act_scales = gs; a.act_sums = gsum;
     a.K = kHidden;
-    a.out = at<float>(ws, p.l.middle);
+    a.mid_words = dw; a.mid_scales = dsc; a.mid_sums = dsum;
     a.silu_table = silu;
     a.sticky = sticky;
-    // above 2048 tokens nearly every tile is full: keep each tile on one XCD
-    a.tile_xcd = T > 2048 ? 1 : 0;
-    TRY(launch_grouped_mfma(a, true, max_tiles, s));
-    auto dw = at<uint32_t>(ws, p.l.down_low);
-    auto dsc = at<uint16_t>(ws, p.l.down_scales);
-    auto dsum = at<int32_t>(ws, p.l.down_sums);
-    // middle rows are in permuted route order; offsets[257] = routes with a valid bank
-    TRY(launch_quant_middle_permuted(at<float>(ws, p.l.middle), RS, ps.offsets + kExperts + 1, qmax, dw, dsc, dsum,
-                                     sticky, s));
+    TRY(launch_grouped_mfma(a, true, qmax, T, max_tiles, s));
     a.codes = static_cast<const uint32_t*>(down_codes);
     a.meta = static_cast<const uint32_t*>(down_meta);
     a.shared_codes = static_cast<const uint32_t*>(sd_codes);
@@ -109,10 +109,8 @@ hipError_t run_routed(const RoutedPlan& p, void* ws, const void* input, const fl
     a.bank_meta_words = kDownBankMeta;
     a.act_words = dw; a.act_scales = dsc; a.act_sums = dsum;
     a.K = kInter;
-    // down: an XCD's m-tiles contiguous up to 2048 tokens (block orders: proj_mfma.hip)
-    a.tile_xcd = T > 2048 ? 0 : 2;
     a.out = at<float>(ws, p.l.route_out);
-    TRY(launch_grouped_mfma(a, false, max_tiles, s));
+    TRY(launch_grouped_mfma(a, false, qmax, T, max_tiles, s));
     return launch_reduce(at<float>(ws, p.l.route_out), weights, ids, T, out ? at<float>(ws, p.l.final_f32) : nullptr,
                          out, shared_logit, shared ? sigmoid : nullptr, shared_out, layer_out, sticky, s);
 }

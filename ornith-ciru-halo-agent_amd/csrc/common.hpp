@@ -476,6 +476,40 @@ __device__ __forceinline__ void quantize_quarter(float v[16], uint32_t words[4],
     sum_out = sum;
 }
 
+// q = clamp(rint(v / scale)) of N values as the bits of kRoundBias + q (q in
+// the low bits, so byte 0 is q's byte).  The quotient is taken as v * rs, rs =
+// RN(1 / scale): in a valid group |v / scale| <= QMAX * (1 + 2^-10) < 128, so
+// the product lies within 2^-16 of v / scale and the correctly rounded
+// quotient within 2^-17 of it; both round to the same integer unless the
+// product lies within 2^-14 of a half-integer (r - rint(r) is exact).  Lanes
+// holding such a value (rare) redo theirs with the correctly rounded division.
+// Adding kRoundBias = 1.5 * 2^23 rounds to the nearest even integer; clamping
+// before it gives what clamping after it gives, the bounds being integers.
+// Values are finite; rs = 0 makes every q zero.
+constexpr float kRoundBias = 12582912.0f;
+template <int QMAX, int N>
+__device__ __forceinline__ void quantize_values(const float (&v)[N], float scale, float rs, uint32_t (&t)[N]) {
+    float far = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float r = __builtin_amdgcn_fmed3f(v[i] * rs, -float(QMAX), float(QMAX));
+        const float b = r + kRoundBias;
+        far = fmaxf(far, fabsf(r - (b - kRoundBias)));
+        t[i] = __float_as_uint(b);
+    }
+    if (far >= 0.5f - 0x1p-14f && rs != 0.f) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float r = __builtin_amdgcn_fmed3f(fdiv_rn(v[i], scale), -float(QMAX), float(QMAX));
+            t[i] = __float_as_uint(r + kRoundBias);
+        }
+    }
+}
+// the low bytes of a, b, c, d, a in the lowest
+__device__ __forceinline__ uint32_t pack_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    return __builtin_amdgcn_perm(b, a, 0x0c0c0400u) | __builtin_amdgcn_perm(d, c, 0x04000c0cu);
+}
+
 // quantize_quarter with the arithmetic of quantize_half_fast (one fma per
 // value detects non-finite values, which OR nonfinite_flags and are zeroed;
 // q = rint(v * RN(1/scale)) with the exact fallback near half-integers):
@@ -505,39 +539,22 @@ __device__ __forceinline__ void quantize_quarter_fast(float v[16], uint32_t word
     const bool zero = absmax == 0.f || !valid;
     const uint16_t sbits = f32_to_f16_bits(zero ? 1.f : fmaxf(raw, 0x1p-14f));
     const float scale = f16_bits_to_f32(sbits);
-    const float rs = fdiv_rn(1.f, scale);
-    float qf[16];
-    bool near = false;
+    const float rs = zero ? 0.f : fdiv_rn(1.f, scale);
+    uint32_t t[16];
+    quantize_values<QMAX>(reinterpret_cast<const float (&)[16]>(*v), scale, rs, t);
+    int sum = 0;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const float r = v[i] * rs;
-        const float n = __builtin_rintf(r);
-        near |= 0.5f - fabsf(r - n) <= 0x1p-14f;
-        qf[i] = n;
-    }
-    if (near) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) qf[i] = __builtin_rintf(fdiv_rn(v[i], scale));
-    }
-    int q[16], sum = 0;
-    const int keep = zero ? 0 : -1;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        q[i] = int(fminf(fmaxf(qf[i], -float(QMAX)), float(QMAX))) & keep;
-        sum += q[i];
+    for (int c = 0; c < 2; ++c) {
+        const uint32_t* tc = t + 8 * c;
+        words[2 * c] = pack_bytes(tc[0], tc[2], tc[4], tc[6]);
+        words[2 * c + 1] = pack_bytes(tc[1], tc[3], tc[5], tc[7]);
+        sum = dot4(int(words[2 * c]), 0x01010101, sum);
+        sum = dot4(int(words[2 * c + 1]), 0x01010101, sum);
     }
     sum += row_ror_i<4>(sum);
     sum += row_ror_i<8>(sum);
     sum += xor_perm_i<1>(sum);
     sum += xor_perm_i<2>(sum);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int* qc = q + 8 * c;
-        words[2 * c] = (uint32_t(qc[0]) & 255u) | ((uint32_t(qc[2]) & 255u) << 8) | ((uint32_t(qc[4]) & 255u) << 16) |
-                       ((uint32_t(qc[6]) & 255u) << 24);
-        words[2 * c + 1] = (uint32_t(qc[1]) & 255u) | ((uint32_t(qc[3]) & 255u) << 8) |
-                           ((uint32_t(qc[5]) & 255u) << 16) | ((uint32_t(qc[7]) & 255u) << 24);
-    }
     sbits_out = sbits;
     sum_out = sum;
 }
@@ -634,37 +651,17 @@ __device__ __forceinline__ void quantize_half_fast(float v[8], uint32_t words[2]
     const bool zero = absmax == 0.f || !valid;
     const uint16_t sbits = f32_to_f16_bits(zero ? 1.f : fmaxf(raw, 0x1p-14f));
     const float scale = f16_bits_to_f32(sbits);
-    const float rs = fdiv_rn(1.f, scale);
-    float qf[8];
-    bool near = false;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float r = v[i] * rs;
-        const float n = __builtin_rintf(r);
-        near |= 0.5f - fabsf(r - n) <= 0x1p-14f;
-        qf[i] = n;
-    }
-    if (near) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) qf[i] = __builtin_rintf(fdiv_rn(v[i], scale));
-    }
-    int q[8], sum = 0;
-    const int keep = zero ? 0 : -1;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int t = int(fminf(fmaxf(qf[i], -float(QMAX)), float(QMAX))) & keep;
-        q[i] = t;
-        sum += t;
-    }
+    const float rs = zero ? 0.f : fdiv_rn(1.f, scale);
+    uint32_t t[8];
+    quantize_values<QMAX>(reinterpret_cast<const float (&)[8]>(*v), scale, rs, t);
+    words[0] = pack_bytes(t[0], t[2], t[4], t[6]);
+    words[1] = pack_bytes(t[1], t[3], t[5], t[7]);
+    int sum = dot4(int(words[1]), 0x01010101, dot4(int(words[0]), 0x01010101, 0));
     sum += xor_perm_i<1>(sum);
     sum += xor_perm_i<2>(sum);
     sum += xor_perm_i<4>(sum);
     sum += xor_perm_i<8>(sum);
     sum += xor_perm_i<16>(sum);
-    words[0] = (uint32_t(q[0]) & 255u) | ((uint32_t(q[2]) & 255u) << 8) | ((uint32_t(q[4]) & 255u) << 16) |
-               ((uint32_t(q[6]) & 255u) << 24);
-    words[1] = (uint32_t(q[1]) & 255u) | ((uint32_t(q[3]) & 255u) << 8) | ((uint32_t(q[5]) & 255u) << 16) |
-               ((uint32_t(q[7]) & 255u) << 24);
     sbits_out = sbits;
     sum_out = sum;
 }

@@ -54,8 +54,8 @@ struct PermuteScratch {
     int32_t* offsets;        // [banks + 1]
     int32_t* routes;         // [routes] permuted route ids
     Segment* segments;       // [banks]
-    int32_t* meta;           // [4]: segment count, mfma tile count, ...
-    Segment* tiles;          // [max tiles] per m-tile: bank, first permuted route, rows, tile-in-segment
+    int32_t* meta;           // [4]: segment count, 64-route tile count, work tile count
+    Segment* tiles;          // [max tiles] per 64-route tile: bank, first permuted route, rows, tile-in-segment
 };
 
 // ---- activations -----------------------------------------------------------
@@ -104,10 +104,12 @@ struct ActJob {
 // when with_shared, routes R..R+T-1 use the shared bank.  act (nullable):
 // that quantisation runs as trailing blocks of the bank-scan launch (its 64
 // blocks leave the rest of the chip idle).
+// work: the projections' m-tiles of work_rows routes, in the form of
+// PermuteScratch::tiles (counted in meta[2]).
 size_t permute_scratch_bytes(int Rcap, int Tcap);
 PermuteScratch carve_permute(void* base, int Rcap, int Tcap);
 hipError_t launch_permute(const int32_t* ids, int R, int T, bool with_shared, const PermuteScratch& p,
-                          uint32_t* sticky, int mfma_rows, hipStream_t s, bool counted = false,
+                          uint32_t* sticky, Segment* work, int work_rows, hipStream_t s, bool counted = false,
                           const ActJob* act = nullptr);
 
 // ---- projections -----------------------------------------------------------
@@ -149,7 +151,9 @@ struct MfmaArgs {
     int64_t bank_words, bank_meta_words;
     const uint32_t* act_words; const uint16_t* act_scales; const int32_t* act_sums;
     int K;
-    float* out;                                  // gate/up: middle [RS, 512]; down: route_out [RS, 2048]
+    float* out;                                  // down: route_out [RS, 2048]
+    // gate/up: the down projection's input [RS, 512] in permuted route order
+    uint32_t* mid_words; uint16_t* mid_scales; int32_t* mid_sums;
     const float* silu_table;
     uint32_t* sticky;
     // dense head (rows = R, identity; columns N): fp32 and bf16 logits [R, N],
@@ -159,17 +163,14 @@ struct MfmaArgs {
     uint16_t* out_bf16;
     float* arg_val; int32_t* arg_idx;
     uint32_t flag_projection, flag_bf16;
-    int tile_xcd;                                // prefill block order: 0 column-block major, 1 tile per XCD, 2 tile ranges per XCD
 };
-hipError_t launch_grouped_mfma(const MfmaArgs& a, bool gateup, int max_tiles, hipStream_t s);
+// gate-up (H128 + quantisation of its middle rows included: mid_*) or down of a layer of T > 32 tokens, whose
+// permutation made m-tiles of grouped_tile_rows(T) rows
+int grouped_tile_rows(int T);
+hipError_t launch_grouped_mfma(const MfmaArgs& a, bool gateup, int qmax, int T, int max_tiles, hipStream_t s);
 // Dense G256 head on the matrix cores: M <= 64 rows of A8 activations against
 // N32 codes, then the per-row argmax (numpy rule) into argmax[M].
 hipError_t launch_head_mfma(const MfmaArgs& a, int64_t* argmax, hipStream_t s);
-// H128 + quantisation of middle rows stored in permuted route order: rows 0 .. *nrows - 1
-// (the permuted routes, all with a valid bank), RS rows at most.
-hipError_t launch_quant_middle_permuted(const float* middle, int RS, const int32_t* nrows, int qmax, uint32_t* words,
-                                        uint16_t* scales, int32_t* sums, uint32_t* sticky, hipStream_t s);
-
 // ---- combination -------------------------------------------------------------
 // out[t] = bf16(sum over valid slots of route_out[8t+s] * w[8t+s]); optional
 // fp32 diagnostic; optional shared output and layer sum.

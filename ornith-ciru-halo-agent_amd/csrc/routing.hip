@@ -29,6 +29,7 @@ __device__ __forceinline__ void bf16x8_to_f32(const uint4 v, float f[8]) {
 
 constexpr int kPermTokens = 16;                      // tokens per permutation count / scatter block
 constexpr int kPermRoutes = kPermTokens * kTop;      // routed routes per block
+constexpr int kTileRoutes = 64;                      // routes per m-tile of the scratch's tile list
 
 // ---------------------------------------------------------------------------
 // Router logits for large T on the matrix cores (declared order above).  A
@@ -582,9 +583,9 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
                                                               int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
                                                               int32_t* __restrict__ routes, Segment* __restrict__ segments,
                                                               int32_t* __restrict__ meta, Segment* __restrict__ tiles,
-                                                              int mfma_rows) {
+                                                              Segment* __restrict__ work, int work_rows) {
     __shared__ int s_off[kBanks + 1];        // exclusive route offsets (s_off[257] = live routes)
-    __shared__ int s_tile[kBanks + 1];       // exclusive m-tile offsets (s_tile[257] = tiles)
+    __shared__ int s_tile[2][kBanks + 1];    // exclusive offsets of the 64-route tiles and the work tiles (at 257: all)
     __shared__ __align__(16) int bank_of[kPermRoutes];
     const int tid = threadIdx.x, lane = tid & 63, R = T * kTop;
     // this thread's route, its bank and the running count of earlier blocks
@@ -600,38 +601,45 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
     if (tid < 64) {
         // bank totals -> offsets, non-empty ranks and m-tile offsets (lane holds
         // banks 4 lane .. 4 lane + 3; the shared bank 256 follows)
-        int tot[4], nt[4], ne[4], part = 0, ntp = 0, nep = 0;
+        int tot[4], nt[4], nw[4], ne[4], part = 0, ntp = 0, nwp = 0, nep = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             tot[i] = counts[4 * lane + i];
-            nt[i] = (tot[i] + mfma_rows - 1) / mfma_rows;
+            nt[i] = (tot[i] + kTileRoutes - 1) / kTileRoutes;
+            nw[i] = (tot[i] + work_rows - 1) / work_rows;
             ne[i] = tot[i] > 0 ? 1 : 0;
             part += tot[i];
             ntp += nt[i];
+            nwp += nw[i];
             nep += ne[i];
         }
         const int incl = wave_inclusive_scan(part), nt_incl = wave_inclusive_scan(ntp);
-        const int ne_incl = wave_inclusive_scan(nep);
-        int off = incl - part, tb = nt_incl - ntp, seg = ne_incl - nep;
+        const int nw_incl = wave_inclusive_scan(nwp), ne_incl = wave_inclusive_scan(nep);
+        int off = incl - part, tb = nt_incl - ntp, wb = nw_incl - nwp, seg = ne_incl - nep;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int e = 4 * lane + i;
             s_off[e] = off;
-            s_tile[e] = tb;
+            s_tile[0][e] = tb;
+            s_tile[1][e] = wb;
             if (blockIdx.x == 0) {
                 offsets[e] = off;
                 if (tot[i] > 0) segments[seg] = Segment{e, off, tot[i], tb};
             }
             off += tot[i];
             tb += nt[i];
+            wb += nw[i];
             seg += ne[i];
         }
         if (lane == 63) {
-            const int snt = (shared_routes + mfma_rows - 1) / mfma_rows;
+            const int snt = (shared_routes + kTileRoutes - 1) / kTileRoutes;
+            const int snw = (shared_routes + work_rows - 1) / work_rows;
             s_off[kExperts] = off;
             s_off[kBanks] = off + shared_routes;
-            s_tile[kExperts] = tb;
-            s_tile[kBanks] = tb + snt;
+            s_tile[0][kExperts] = tb;
+            s_tile[0][kBanks] = tb + snt;
+            s_tile[1][kExperts] = wb;
+            s_tile[1][kBanks] = wb + snw;
             if (blockIdx.x == 0) {
                 offsets[kExperts] = off;
                 offsets[kBanks] = off + shared_routes;
@@ -639,22 +647,27 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
                 if (shared_routes > 0) segments[seg] = Segment{kExperts, off, shared_routes, tb};
                 meta[0] = seg + (shared_routes > 0 ? 1 : 0);
                 meta[1] = tb + snt;
+                meta[2] = wb + snw;
             }
         }
     }
     __syncthreads();
-    // m-tiles, spread over the grid: tile i belongs to the bank e with
-    // s_tile[e] <= i < s_tile[e + 1] (binary search; empty banks have no tiles)
-    const int ntiles = s_tile[kBanks];
-    for (int i = blockIdx.x * 256 + tid; i < ntiles; i += gridDim.x * 256) {
-        int lo = 0, hi = kBanks;                    // s_tile[lo] <= i < s_tile[hi]
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (s_tile[mid] <= i) lo = mid; else hi = mid;
+    // m-tiles of both lists, spread over the grid: tile i belongs to the bank e
+    // with s_tile[e] <= i < s_tile[e + 1] (binary search; empty banks have none)
+    auto list = [&](const int* first_tile, Segment* out, int rows) {
+        const int ntiles = first_tile[kBanks];
+        for (int i = blockIdx.x * 256 + tid; i < ntiles; i += gridDim.x * 256) {
+            int lo = 0, hi = kBanks;                // first_tile[lo] <= i < first_tile[hi]
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (first_tile[mid] <= i) lo = mid; else hi = mid;
+            }
+            const int k = i - first_tile[lo], total = s_off[lo + 1] - s_off[lo];
+            out[i] = Segment{lo, s_off[lo] + k * rows, min(rows, total - k * rows), k};
         }
-        const int k = i - s_tile[lo], total = s_off[lo + 1] - s_off[lo];
-        tiles[i] = Segment{lo, s_off[lo] + k * mfma_rows, min(mfma_rows, total - k * mfma_rows), k};
-    }
+    };
+    list(s_tile[0], tiles, kTileRoutes);
+    list(s_tile[1], work, work_rows);
     if (tid < kPermRoutes && b >= 0) {
         // rank in the block = earlier routes of the block with bank b: all of
         // an earlier token's eight, the first `slot` of this token's (a token
@@ -678,7 +691,8 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
 }
 
 hipError_t launch_permute(const int32_t* ids, int R, int T, bool with_shared, const PermuteScratch& p,
-                          uint32_t* sticky, int mfma_rows, hipStream_t s, bool counted, const ActJob* act) {
+                          uint32_t* sticky, Segment* work, int work_rows, hipStream_t s, bool counted,
+                          const ActJob* act) {
     if (R != T * kTop) return hipErrorInvalidValue;
     const int nblocks = (T + kPermTokens - 1) / kPermTokens;
     if (nblocks > 8 * 64) return hipErrorInvalidValue;
@@ -701,7 +715,7 @@ hipError_t launch_permute(const int32_t* ids, int R, int T, bool with_shared, co
     if (st != hipSuccess) return st;
     timed_launch("permute_scatter", permute_scatter_kernel, dim3(nblocks), dim3(256), 0, s, ids, T,
                  with_shared ? T : 0, p.block_counts, p.counts, p.offsets, p.routes, p.segments, p.meta, p.tiles,
-                 mfma_rows);
+                 work, work_rows);
     return hipGetLastError();
 }
 
