@@ -73,10 +73,15 @@ hipError_t launch_act_middle(const float* gate_y, int RS, int R, const int32_t* 
                              int32_t* sums, uint32_t* sticky, hipStream_t s);
 
 // ---- routing ---------------------------------------------------------------
-constexpr int kRouterRowsMaxTokens = 256;      // wave-per-row router up to here, token-tiled beyond
+// Wave-per-row router up to here, token-tiled beyond: rows against tiles 10.2 /
+// 13.4 us at 96 tokens, 13.3 / 13.3 at 131, 14.4 / 13.3 at 160, 20.0 / 13.4 at
+// 256 (the tile kernel's blocks are all resident up to 1024 tokens, so its time
+// hardly moves).
+constexpr int kRouterRowsMaxTokens = 144;
+constexpr int kRouterSplitMinTokens = 256;     // the split tail (and its scratch) only beyond
 // Router logits [T, 256 (+1)] in the declared order; shared_w (nullable) adds
 // column 256, the shared-expert gate logit.  split_sums (nullable,
-// router_split_bytes): for T > kRouterRowsMaxTokens the last
+// router_split_bytes): for T > kRouterSplitMinTokens the last
 // router_split_groups(T) token groups run as eighth-tile units whose partial
 // sums launch_topk completes (their logits are final only after it).
 hipError_t launch_router(const uint16_t* x, int64_t stride, int T, const uint16_t* w, const uint16_t* shared_w,

@@ -353,7 +353,7 @@ hipError_t launch_router(const uint16_t* x, int64_t stride, int T, const uint16_
 // its loads' latency besides an eighth of a tile's products, so larger
 // remainders stay whole tiles).
 int router_split_groups(int T) {
-    if (T <= kRouterRowsMaxTokens) return 0;
+    if (T <= kRouterSplitMinTokens) return 0;
     const int cus = device_cu_count(), per = cus / 8, ntg = (T + kRmTile - 1) / kRmTile;
     if (per <= 0 || ntg < per) return 0;
     const int left = ntg % per;
@@ -361,7 +361,7 @@ int router_split_groups(int T) {
 }
 
 size_t router_split_bytes(int Tcap) {
-    if (Tcap <= kRouterRowsMaxTokens) return 0;
+    if (Tcap <= kRouterSplitMinTokens) return 0;
     const int groups = std::max(1, 2 * device_cu_count() / 64);
     return size_t(groups) * 64 * kRmTile * kRmTile * sizeof(float);
 }
