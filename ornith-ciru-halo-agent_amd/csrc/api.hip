@@ -66,15 +66,17 @@ hipError_t run_routed(const RoutedPlan& p, void* ws, const void* input, const fl
     const bool shared = sg_codes != nullptr;
     const int R = T * kTop, RS = R + (shared ? T : 0);
     const PermuteScratch ps = carve_permute(at<void>(ws, p.permute), Tcap * kTop, shared ? Tcap : 0);
-    // the projections' m-tiles are listed in the (otherwise unused) gate_y rows, 4 KiB a route
-    Segment* work = at<Segment>(ws, p.l.gate_y);
+    // the (otherwise unused) gate_y rows, 4 KiB a route, hold the raw block counts (64 bytes a token, 1 KiB at
+    // least) and the projections' m-tiles
+    int32_t* raw = at<int32_t>(ws, p.l.gate_y);
+    Segment* work = at<Segment>(raw, align256(size_t(T) * 64 + 1024));
     const int tile_rows = grouped_tile_rows(T);
     auto gw = at<uint32_t>(ws, p.l.gate_low);
     auto gs = at<uint16_t>(ws, p.l.gate_scales);
     auto gsum = at<int32_t>(ws, p.l.gate_sums);
     // the A8 gate input rides on the bank-scan launch (the A4 one has its own)
     const ActJob act{static_cast<const uint16_t*>(input), T, shared ? nullptr : ids, gw, gs, gsum};
-    TRY(launch_permute(ids, R, T, shared, ps, sticky, work, tile_rows, s, counted, qmax == 127 ? &act : nullptr));
+    TRY(launch_permute(ids, R, T, shared, ps, sticky, work, tile_rows, raw, s, counted, qmax == 127 ? &act : nullptr));
     if (qmax != 127)
         TRY(launch_act_bf16(static_cast<const uint16_t*>(input), kHidden, T, kHidden, qmax, shared ? nullptr : ids, gw,
                             gs, gsum, sticky, kFlagNonfiniteInput, kFlagInvalidActivation, s));
@@ -369,7 +371,8 @@ extern "C" hipError_t ornith_moe_layer_launch(
                       static_cast<const uint16_t*>(shared_gate_w), static_cast<const float*>(bias), logits,
                       kLogitStride, stream, split));
     TRY(launch_topk(logits, kLogitStride, T, static_cast<float*>(topk_weights), static_cast<int32_t*>(topk_ids),
-                    logits + kExperts, kLogitStride, static_cast<uint16_t*>(shared_logit), stream, ps.block_counts,
+                    logits + kExperts, kLogitStride, static_cast<uint16_t*>(shared_logit), stream,
+                    permute_fused(T) ? at<int32_t>(workspace, p.l.gate_y) : ps.block_counts,
                     split, static_cast<const float*>(bias)));
     return run_routed(p, workspace, input, static_cast<const float*>(topk_weights),
                       static_cast<const int32_t*>(topk_ids), gate_codes, gate_meta, down_codes, down_meta,

@@ -109,12 +109,18 @@ struct ActJob {
 // when with_shared, routes R..R+T-1 use the shared bank.  act (nullable):
 // that quantisation runs as trailing blocks of the bank-scan launch (its 64
 // blocks leave the rest of the chip idle).
+// Up to kPermFusedBlocks 16-token blocks the bank scan is part of the scatter
+// launch (and act's blocks with it): one launch less, every block reading the
+// other blocks' 1 KiB of counts.  The count step then writes to `raw`
+// ([blocks, 256]) instead of block_counts.
+constexpr int kPermFusedBlocks = 128;
+inline bool permute_fused(int T) { return (T + 15) / 16 <= kPermFusedBlocks; }
 // work: the projections' m-tiles of work_rows routes, in the form of
 // PermuteScratch::tiles (counted in meta[2]).
 size_t permute_scratch_bytes(int Rcap, int Tcap);
 PermuteScratch carve_permute(void* base, int Rcap, int Tcap);
 hipError_t launch_permute(const int32_t* ids, int R, int T, bool with_shared, const PermuteScratch& p,
-                          uint32_t* sticky, Segment* work, int work_rows, hipStream_t s, bool counted = false,
+                          uint32_t* sticky, Segment* work, int work_rows, int32_t* raw, hipStream_t s, bool counted = false,
                           const ActJob* act = nullptr);
 
 // ---- projections -----------------------------------------------------------

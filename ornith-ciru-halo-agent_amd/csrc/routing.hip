@@ -517,7 +517,8 @@ PermuteScratch carve_permute(void* base, int Rcap, int Tcap) {
 //   count      per 16-token block, the routed banks' route counts (LDS
 //              histogram; fused into topk_kernel on the layer path)
 //   bank scan  one wave per routed bank: exclusive running sums over blocks
-//              (in place) and the bank total
+//              (in place) and the bank total; with few blocks each scatter
+//              block forms its own sums instead
 //   scatter    every block scans the 257 bank totals into offsets; block 0
 //              also writes offsets, segments, the MFMA tile list and meta; a
 //              route's slot is offset + running sum + its rank in the block.
@@ -578,15 +579,30 @@ __global__ __launch_bounds__(256) void permute_bank_scan_act_kernel(int nblocks,
                             act.scales, act.sums, sticky, kFlagNonfiniteInput, kFlagInvalidActivation);
 }
 
+// FUSED (at most kPermFusedBlocks blocks): raw holds the blocks' counts as the
+// count step left them; every block sums all of them for itself (its running
+// counts and the totals), and the blocks past nblocks run the activation
+// quantisation (act_bf16_block indices 0, 1, ...).  Otherwise the bank scan has
+// left running counts in block_counts and totals in counts.
+template <bool FUSED>
 __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __restrict__ ids, int T, int shared_routes,
-                                                              const int32_t* __restrict__ block_counts,
+                                                              int nblocks, const int32_t* __restrict__ raw,
+                                                              int32_t* __restrict__ block_counts,
                                                               int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
                                                               int32_t* __restrict__ routes, Segment* __restrict__ segments,
                                                               int32_t* __restrict__ meta, Segment* __restrict__ tiles,
-                                                              Segment* __restrict__ work, int work_rows) {
+                                                              Segment* __restrict__ work, int work_rows, ActJob act,
+                                                              uint32_t* sticky) {
     __shared__ int s_off[kBanks + 1];        // exclusive route offsets (s_off[257] = live routes)
     __shared__ int s_tile[2][kBanks + 1];    // exclusive offsets of the 64-route tiles and the work tiles (at 257: all)
     __shared__ __align__(16) int bank_of[kPermRoutes];
+    __shared__ __align__(16) int s_total[FUSED ? kExperts : 1];
+    __shared__ int s_before[FUSED ? kExperts : 1];
+    if (FUSED && int(blockIdx.x) >= nblocks) {
+        act_bf16_block<127>(int(blockIdx.x) - nblocks, act.x, kHidden, act.rows, kHidden / kGroup, act.ids, act.words,
+                            act.scales, act.sums, sticky, kFlagNonfiniteInput, kFlagInvalidActivation);
+        return;
+    }
     const int tid = threadIdx.x, lane = tid & 63, R = T * kTop;
     // this thread's route, its bank and the running count of earlier blocks
     // (loaded before the offsets are ready)
@@ -595,8 +611,26 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
     int b = -1, before = 0;
     if (tid < kPermRoutes) {
         b = r < R ? route_bank(ids, r, R, dummy) : -1;
-        if (b >= 0) before = block_counts[size_t(blockIdx.x) * kExperts + b];
+        if (!FUSED && b >= 0) before = block_counts[size_t(blockIdx.x) * kExperts + b];
         bank_of[tid] = b;
+    }
+    if constexpr (FUSED) {
+        int total = 0, earlier = 0;                            // thread = bank
+        for (int k0 = 0; k0 < nblocks; k0 += 32) {             // 32 blocks' counts in flight at once
+            int v[32];
+#pragma unroll
+            for (int k = 0; k < 32; ++k) v[k] = raw[min(k0 + k, nblocks - 1) * kExperts + tid];
+#pragma unroll
+            for (int k = 0; k < 32; ++k) {
+                total += k0 + k < nblocks ? v[k] : 0;
+                earlier += k0 + k < int(blockIdx.x) ? v[k] : 0;
+            }
+        }
+        s_total[tid] = total;
+        s_before[tid] = earlier;
+        block_counts[size_t(blockIdx.x) * kExperts + tid] = earlier;
+        if (blockIdx.x == 0) counts[tid] = total;
+        __syncthreads();
     }
     if (tid < 64) {
         // bank totals -> offsets, non-empty ranks and m-tile offsets (lane holds
@@ -604,7 +638,7 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
         int tot[4], nt[4], nw[4], ne[4], part = 0, ntp = 0, nwp = 0, nep = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            tot[i] = counts[4 * lane + i];
+            tot[i] = FUSED ? s_total[4 * lane + i] : counts[4 * lane + i];
             nt[i] = (tot[i] + kTileRoutes - 1) / kTileRoutes;
             nw[i] = (tot[i] + work_rows - 1) / work_rows;
             ne[i] = tot[i] > 0 ? 1 : 0;
@@ -656,7 +690,7 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
     // with s_tile[e] <= i < s_tile[e + 1] (binary search; empty banks have none)
     auto list = [&](const int* first_tile, Segment* out, int rows) {
         const int ntiles = first_tile[kBanks];
-        for (int i = blockIdx.x * 256 + tid; i < ntiles; i += gridDim.x * 256) {
+        for (int i = blockIdx.x * 256 + tid; i < ntiles; i += nblocks * 256) {
             int lo = 0, hi = kBanks;                // first_tile[lo] <= i < first_tile[hi]
             while (hi - lo > 1) {
                 const int mid = (lo + hi) >> 1;
@@ -668,6 +702,7 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
     };
     list(s_tile[0], tiles, kTileRoutes);
     list(s_tile[1], work, work_rows);
+    if (FUSED && b >= 0) before = s_before[b];
     if (tid < kPermRoutes && b >= 0) {
         // rank in the block = earlier routes of the block with bank b: all of
         // an earlier token's eight, the first `slot` of this token's (a token
@@ -691,31 +726,40 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
 }
 
 hipError_t launch_permute(const int32_t* ids, int R, int T, bool with_shared, const PermuteScratch& p,
-                          uint32_t* sticky, Segment* work, int work_rows, hipStream_t s, bool counted,
+                          uint32_t* sticky, Segment* work, int work_rows, int32_t* raw, hipStream_t s, bool counted,
                           const ActJob* act) {
     if (R != T * kTop) return hipErrorInvalidValue;
     const int nblocks = (T + kPermTokens - 1) / kPermTokens;
     if (nblocks > 8 * 64) return hipErrorInvalidValue;
+    const bool fused = nblocks <= kPermFusedBlocks;
+    if (fused && !raw) return hipErrorInvalidValue;
+    int32_t* step1 = fused ? raw : p.block_counts;
     if (!counted) {
-        timed_launch("permute_count", permute_count_kernel, dim3(nblocks), dim3(kPermRoutes), 0, s, ids, T,
-                     p.block_counts, sticky);
+        timed_launch("permute_count", permute_count_kernel, dim3(nblocks), dim3(kPermRoutes), 0, s, ids, T, step1,
+                     sticky);
         const hipError_t st = hipGetLastError();
         if (st != hipSuccess) return st;
     }
-    if (act) {
-        // act_bf16_block: four 4-group waves per block index
-        const int act_blocks = (act->rows * (kHidden / kGroup) + 15) / 16;
+    // act_bf16_block: four 4-group waves per block index
+    const int act_blocks = act ? (act->rows * (kHidden / kGroup) + 15) / 16 : 0;
+    const ActJob job = act ? *act : ActJob{};
+    if (fused) {
+        timed_launch("permute_scatter_act", permute_scatter_kernel<true>, dim3(nblocks + act_blocks), dim3(256), 0, s,
+                     ids, T, with_shared ? T : 0, nblocks, raw, p.block_counts, p.counts, p.offsets, p.routes,
+                     p.segments, p.meta, p.tiles, work, work_rows, job, sticky);
+        return hipGetLastError();
+    }
+    if (act)
         timed_launch("permute_scan_act", permute_bank_scan_act_kernel, dim3(kExperts / 4 + act_blocks), dim3(256), 0,
-                     s, nblocks, p.block_counts, p.counts, *act, sticky);
-    } else {
+                     s, nblocks, p.block_counts, p.counts, job, sticky);
+    else
         timed_launch("permute_scan", permute_bank_scan_kernel, dim3(kExperts / 4), dim3(256), 0, s, nblocks,
                      p.block_counts, p.counts);
-    }
     hipError_t st = hipGetLastError();
     if (st != hipSuccess) return st;
-    timed_launch("permute_scatter", permute_scatter_kernel, dim3(nblocks), dim3(256), 0, s, ids, T,
-                 with_shared ? T : 0, p.block_counts, p.counts, p.offsets, p.routes, p.segments, p.meta, p.tiles,
-                 work, work_rows);
+    timed_launch("permute_scatter", permute_scatter_kernel<false>, dim3(nblocks), dim3(256), 0, s, ids, T,
+                 with_shared ? T : 0, nblocks, static_cast<const int32_t*>(nullptr), p.block_counts, p.counts,
+                 p.offsets, p.routes, p.segments, p.meta, p.tiles, work, work_rows, job, sticky);
     return hipGetLastError();
 }
 
