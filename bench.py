@@ -51,12 +51,11 @@ DENSE_N = 6144
 MEASURED_TRAFFIC = {
     ('layer1', 1): 16768264, ('route1', 1): 1166652, ('gateup1', 1): 9949504, ('down1', 1): 5118494,
     ('route_select', 32): 5329307, ('gateup', 32): 176476340, ('down', 32): 94490777, ('reduce', 32): 2596402,
-    ('router', 1120): 15343263, ('topk', 1120): 2186638, ('permute_scan_act', 1120): 7786592,
-    ('permute_scatter', 1120): 320474, ('gateup_mfma', 1120): 190732263, ('quant_middle', 1120): 26020249,
-    ('down_mfma', 1120): 177260462, ('reduce', 1120): 87590525,
-    ('router', 8192): 50519818, ('topk', 8192): 9599320, ('permute_scan_act', 8192): 56100945,
-    ('permute_scatter', 8192): 1531030, ('gateup_mfma', 8192): 625504138,
-    ('quant_middle', 8192): 189713102, ('down_mfma', 8192): 845063402, ('reduce', 8192): 639829271,
+    ('router', 1120): 15343159, ('topk', 1120): 2186694, ('permute_scatter_act', 1120): 7971476,
+    ('gateup_mfma', 1120): 137523438, ('down_mfma', 1120): 146047665, ('reduce', 1120): 87588630,
+    ('router', 8192): 50519792, ('topk', 8192): 9599227, ('permute_scan_act', 8192): 56091210,
+    ('permute_scatter', 8192): 1569102, ('gateup_mfma', 8192): 320505027, ('down_mfma', 8192): 709583375,
+    ('reduce', 8192): 639837397,
 }
 
 
@@ -79,7 +78,7 @@ def kernel_cost(name, T, unique):
     if name in ('down1', 'down'):
         return 'hbm', banks * DOWN_BYTES + routes * 512 * 4 + T * 2048 * 2, HBM_PEAK_GBS, 'GB/s'
     if name in ('gateup_mfma', 'down_mfma'):
-        if name == 'gateup_mfma':       # codes + meta, A8 gate input in, fp32 middle rows out
+        if name == 'gateup_mfma':       # codes + meta, A8 gate input in, middle rows out (priced as fp32)
             nbytes, ops = banks * GATEUP_BYTES + T * 2048 + routes * 512 * 4, 2 * routes * 1024 * 2048
         else:                           # codes + meta, A8 middle rows in, fp32 route rows out
             nbytes, ops = banks * DOWN_BYTES + routes * 512 + routes * 2048 * 4, 2 * routes * 2048 * 512
@@ -88,7 +87,7 @@ def kernel_cost(name, T, unique):
         return 'mfma', ops, INT8_PEAK_TOPS, 'TFLOP/s'
     if name == 'router':      # exact K=1 fp32 matrix steps (the shared-gate row on the VALU)
         return 'mfma', 2 * T * 257 * 2048, FP32_PEAK_TFLOPS, 'TFLOP/s'
-    if name == 'permute_scan_act':  # the scan's block counts are noise beside the gate-input quantisation
+    if name in ('permute_scan_act', 'permute_scatter_act'):  # the block counts are noise beside the quantisation
         return 'hbm', T * 2048 * 2 + T * 2048 + T * 8 * (2 + 4), HBM_PEAK_GBS, 'GB/s'
     return 'hbm', T * 2048 * 2, HBM_PEAK_GBS, 'GB/s'
 

@@ -510,10 +510,12 @@ __device__ __forceinline__ uint32_t pack_bytes(uint32_t a, uint32_t b, uint32_t 
     return __builtin_amdgcn_perm(b, a, 0x0c0c0400u) | __builtin_amdgcn_perm(d, c, 0x04000c0cu);
 }
 
-// quantize_quarter with the arithmetic of quantize_half_fast (one fma per
-// value detects non-finite values, which OR nonfinite_flags and are zeroed;
-// q = rint(v * RN(1/scale)) with the exact fallback near half-integers):
-// the same words, scale and sum.
+// quantize_quarter with fewer operations (one fma per value detects non-finite
+// values, which OR nonfinite_flags and are zeroed; quantize_values): the same
+// words, scale and sum.  The half-wave form below keeps separate conversions:
+// its kernels wait on one group's chain, where the running maximum of
+// quantize_values costs more than the instructions it saves (single-token layer
+// +1 %).
 template <int QMAX>
 __device__ __forceinline__ void quantize_quarter_fast(float v[16], uint32_t words[4], uint16_t& sbits_out,
                                                       int& sum_out, uint32_t& flags, uint32_t nonfinite_flags,
@@ -651,17 +653,37 @@ __device__ __forceinline__ void quantize_half_fast(float v[8], uint32_t words[2]
     const bool zero = absmax == 0.f || !valid;
     const uint16_t sbits = f32_to_f16_bits(zero ? 1.f : fmaxf(raw, 0x1p-14f));
     const float scale = f16_bits_to_f32(sbits);
-    const float rs = zero ? 0.f : fdiv_rn(1.f, scale);
-    uint32_t t[8];
-    quantize_values<QMAX>(reinterpret_cast<const float (&)[8]>(*v), scale, rs, t);
-    words[0] = pack_bytes(t[0], t[2], t[4], t[6]);
-    words[1] = pack_bytes(t[1], t[3], t[5], t[7]);
-    int sum = dot4(int(words[1]), 0x01010101, dot4(int(words[0]), 0x01010101, 0));
+    const float rs = fdiv_rn(1.f, scale);
+    float qf[8];
+    bool near = false;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float r = v[i] * rs;
+        const float n = __builtin_rintf(r);
+        near |= 0.5f - fabsf(r - n) <= 0x1p-14f;
+        qf[i] = n;
+    }
+    if (near) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) qf[i] = __builtin_rintf(fdiv_rn(v[i], scale));
+    }
+    int q[8], sum = 0;
+    const int keep = zero ? 0 : -1;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int t = int(fminf(fmaxf(qf[i], -float(QMAX)), float(QMAX))) & keep;
+        q[i] = t;
+        sum += t;
+    }
     sum += xor_perm_i<1>(sum);
     sum += xor_perm_i<2>(sum);
     sum += xor_perm_i<4>(sum);
     sum += xor_perm_i<8>(sum);
     sum += xor_perm_i<16>(sum);
+    words[0] = (uint32_t(q[0]) & 255u) | ((uint32_t(q[2]) & 255u) << 8) | ((uint32_t(q[4]) & 255u) << 16) |
+               ((uint32_t(q[6]) & 255u) << 24);
+    words[1] = (uint32_t(q[1]) & 255u) | ((uint32_t(q[3]) & 255u) << 8) | ((uint32_t(q[5]) & 255u) << 16) |
+               ((uint32_t(q[7]) & 255u) << 24);
     sbits_out = sbits;
     sum_out = sum;
 }
