@@ -462,10 +462,10 @@ hipError_t launch_grouped_mfma(const MfmaArgs& a, bool gateup, int qmax, int T, 
     //    are read once and bypass the caches (48 tokens: gate-up 42.5 -> 41.6
     //    us, down 24.4 -> 23.2); beyond, skewed routing re-reads them (512
     //    tokens, Zipf 1.1: 37.6 against 48.6 us) and plain loads are better;
-    //  - down blocks of 1024 columns repeat the row staging less, blocks of 512
-    //    fill the chip better in between: 131 tokens 33.4 against 34.8 us with
-    //    the former once the codes bypass the caches, 1120 tokens 39 against
-    //    41 us with the latter, 8192 tokens 199 against 212 us with the former.
+    //  - down blocks cover 1024 columns at both ends, 512 in between: the larger
+    //    stage the rows half as often (8192 tokens 199 against 212 us, 48 tokens
+    //    23.2 against 27.1), the smaller fill the chip better (1120 tokens 39
+    //    against 41 us).
     if (T <= 64) return launch_tiles<16, 8, 4, 4, true>(a, gateup, qmax, max_tiles, s);
     if (grouped_tile_rows(T) == 16) return launch_tiles<16, 8, 4, 2, false>(a, gateup, qmax, max_tiles, s);
     if (T <= 2048) return launch_tiles<32, 4, 4, 2, false>(a, gateup, qmax, max_tiles, s);
