@@ -449,8 +449,16 @@ hipError_t launch_tiles(const MfmaArgs& a, bool gateup, int qmax, int max_tiles,
 // codes and unpack them half as often (two waves per SIMD).  Layer time, 16
 // against 32 rows: N32 banks 135 / 147 us at 256 tokens, 148 / 153 at 512,
 // 171 / 158 at 700 (even routing), 149 / 143 at 1120 (Zipf 1.1); N16 banks
-// (routed projections alone) 103 / 106 at 80, 130 / 120 at 300.
-int grouped_tile_rows(int T) { return T <= (kRoutedTile == 32 ? 512 : 192) ? 16 : 32; }
+// (routed projections alone) 103 / 106 at 80, 130 / 128 at 400, 139 / 135 at
+// 550.  With N16 banks 16-row tiles come back where an even share (T / 32
+// routes) comes close to 32: a few experts beyond it put the 32-row blocks just
+// past one round of the chip's 512 slots (even routing 144 / 159 at 700, 153 /
+// 163 at 900; Zipf 1.2 91 / 86 at 700), until two tiles an expert are the rule
+// (167 / 164 at 1100).
+int grouped_tile_rows(int T) {
+    if (kRoutedTile == 32) return T <= 512 ? 16 : 32;
+    return T <= 192 || (T > 576 && T <= 1024) ? 16 : 32;
+}
 
 hipError_t launch_grouped_mfma(const MfmaArgs& a, bool gateup, int qmax, int T, int max_tiles, hipStream_t s) {
     if (max_tiles <= 0) return hipSuccess;
