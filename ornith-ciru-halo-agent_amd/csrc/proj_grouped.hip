@@ -137,8 +137,9 @@ __device__ __forceinline__ void stage_rows(Rows<MT, GS>& R, const MfmaArgs& a) {
 // Dots and fp32 tree of one 256-group for L row tiles of 16 rows.
 // val[rt][ct][r]: row 16 rt + 4 q + r, column ct of the lane.  Each k-step's
 // words are refilled with group gnext of `next` as soon as they are unpacked,
-// so a wave always has about 8 KiB of codes in flight.
-template <int L, bool ONCE, int MT, int GS, int TW>
+// so a wave always has about 8 KiB of codes in flight (REFILL false: the
+// wave's last step, nothing is left to load).
+template <int L, bool ONCE, bool REFILL = true, int MT, int GS, int TW>
 __device__ __forceinline__ void group_step(const Rows<MT, GS>& R, Codes& c, int g, float (&val)[L][4][4],
                                            const BankLane<TW>& next, int gnext) {
     const int lane = threadIdx.x & 63, li = lane & 15, q = lane >> 4;
@@ -154,7 +155,7 @@ __device__ __forceinline__ void group_step(const Rows<MT, GS>& R, Codes& c, int 
         i32x4 fb[4];
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct) fb[ct] = b_operand(c, s, ct);
-        next.template load<ONCE>(c, s, gnext);
+        if constexpr (REFILL) next.template load<ONCE>(c, s, gnext);
 #pragma unroll
         for (int rt = 0; rt < L; ++rt) {
             const u32x4 v =
@@ -165,7 +166,7 @@ __device__ __forceinline__ void group_step(const Rows<MT, GS>& R, Codes& c, int 
                 acc[rt][ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa, fb[ct], s ? acc[rt][ct] : kInit, 0, 0, 0);
         }
     }
-    next.load_meta(c, gnext);
+    if constexpr (REFILL) next.load_meta(c, gnext);
 #pragma unroll
     for (int rt = 0; rt < L; ++rt) {
         // RN(offset * RN(sa * sum)) of the lane's four columns x four rows by
@@ -362,11 +363,19 @@ gateup_tile_kernel(MfmaArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Down: block (m-tile, CH x 512 columns); wave w's chunk c is columns
-// 512 (CH nt + c) + 64 w .. + 63.  Both groups (K = 512) of the rows are in LDS.
+// Down: block (m-tile, CH x 256 columns); wave w's chunk c is columns
+// 256 (CH nt + c) + 64 w .. + 63.  Both groups (K = 512) of the rows are in LDS.
+// Bound by the code stream at few tokens and by the fp32 route rows it writes
+// at many (604 MB at 8192 tokens with the shared expert), so it wants waves in
+// flight: 16-row blocks stay within 128 registers without scratch (four waves
+// per SIMD), 32-row ones within 168 (three), which one loop over the group
+// steps allows (unrolled by group it needs 230 and spills at 16 rows).  The
+// wave's last step is outside the loop: it has no codes left to load.  With two
+// waves per SIMD, 24 bytes of scratch at 16 rows and that refill of codes
+// nobody used: 36.7 -> 32.2 us at 131 tokens, 68.3 -> 60.7 at 2048.
 // ---------------------------------------------------------------------------
 template <int MT, int WAVES, int CH, bool ONCE>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(MT == 16 ? 4 : 2, MT == 16 ? 4 : 2))) void
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(MT == 16 ? 4 : 3, MT == 16 ? 4 : 3))) void
 down_tile_kernel(MfmaArgs a) {
     constexpr int GS = kInter / kGroup, kCols = 64 * WAVES, NCB = kHidden / (kCols * CH);
     __shared__ __attribute__((aligned(16))) Rows<MT, GS> R;
@@ -393,18 +402,14 @@ down_tile_kernel(MfmaArgs a) {
         stage_rows<MT, GS, 64 * WAVES>(R, a);
         __syncthreads();
         auto run = [&]<int L>() {
-#pragma unroll 1
-            for (int ch = 0; ch < CH; ++ch) {
-                float val[L][4][4];
+            float val[L][4][4];
 #pragma unroll
-                for (int rt = 0; rt < L; ++rt)
+            for (int rt = 0; rt < L; ++rt)
 #pragma unroll
-                    for (int ct = 0; ct < 4; ++ct)
+                for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) val[rt][ct][r] = 0.f;
-#pragma unroll 1
-                for (int g = 0; g < GS; ++g)               // GS = 2: the other group, then the next chunk's first
-                    group_step<L, ONCE>(R, c, g, val, bank_at.ahead(kCols * min(ch + g, CH - 1), GS), 1 - g);
+                    for (int r = 0; r < 4; ++r) val[rt][ct][r] = 0.f;
+            auto finish = [&](int ch) {
 #pragma unroll
                 for (int rt = 0; rt < L; ++rt)
 #pragma unroll
@@ -414,11 +419,20 @@ down_tile_kernel(MfmaArgs a) {
                         for (int ct = 0; ct < 4; ++ct) {
                             v[ct] = shared ? bf16_round(val[rt][ct][r]) : val[rt][ct][r];
                             nonfinite = __builtin_fmaf(v[ct], 0.f, nonfinite);
+                            val[rt][ct][r] = 0.f;
                         }
                         const int to = R.route[16 * rt + 4 * q + r];
                         if (to >= 0) *reinterpret_cast<f32x4*>(a.out + size_t(to) * kHidden + col0 + kCols * ch) = v;
                     }
+            };
+            // step st: group st % 2 of chunk st / 2 (GS = 2), refilled with the next step's codes
+#pragma unroll 1
+            for (int st = 0; st < 2 * CH - 1; ++st) {
+                group_step<L, ONCE>(R, c, st & 1, val, bank_at.ahead(kCols * ((st + 1) >> 1), GS), (st + 1) & 1);
+                if (st & 1) finish(st >> 1);
             }
+            group_step<L, ONCE, false>(R, c, 1, val, bank_at, 0);
+            finish(CH - 1);
         };
         if (MT > 16 && nrows > 16) run.template operator()<MT / 16>();
         else run.template operator()<1>();
@@ -470,13 +484,17 @@ hipError_t launch_grouped_mfma(const MfmaArgs& a, bool gateup, int qmax, int T, 
     //    are read once and bypass the caches (48 tokens: gate-up 42.5 -> 41.6
     //    us, down 24.4 -> 23.2); beyond, skewed routing re-reads them (512
     //    tokens, Zipf 1.1: 37.6 against 48.6 us) and plain loads are better;
-    //  - down blocks cover 1024 columns at both ends, 512 in between: the larger
-    //    stage the rows half as often (8192 tokens 199 against 212 us, 48 tokens
-    //    23.2 against 27.1), the smaller fill the chip better (1120 tokens 39
-    //    against 41 us).
-    if (T <= 64) return launch_tiles<16, 8, 4, 4, true>(a, gateup, qmax, max_tiles, s);
+    //  - down blocks cover 256 columns up to 64 tokens, where few experts leave
+    //    the chip empty (Zipf 1.1, 256 / 512 / 1024 columns: 33 tokens 8.7 /
+    //    10.1 / 13.6 us, 64 tokens 9.8 / 10.9 / 14.3; evenly routed 24.0 / 24.3 /
+    //    24.1), 512 beyond (1120 tokens 37 us against 39 with 1024, 64 with
+    //    256), and 1024 where every expert has several tiles and staging the rows
+    //    half as often counts for more than the extra blocks (even routing, N16
+    //    banks, 512 / 1024 columns: 2100 tokens 58.0 / 60.1, 4000 97.0 / 93.8,
+    //    8192 191 / 178; Zipf 1.1: 53.8 / 57.3, 91.3 / 95.6, 173.6 / 170.8).
+    if (T <= 64) return launch_tiles<16, 8, 4, 1, true>(a, gateup, qmax, max_tiles, s);
     if (grouped_tile_rows(T) == 16) return launch_tiles<16, 8, 4, 2, false>(a, gateup, qmax, max_tiles, s);
-    if (T <= 2048) return launch_tiles<32, 4, 4, 2, false>(a, gateup, qmax, max_tiles, s);
+    if (T <= 5120) return launch_tiles<32, 4, 4, 2, false>(a, gateup, qmax, max_tiles, s);
     return launch_tiles<32, 4, 4, 4, false>(a, gateup, qmax, max_tiles, s);
 }
 

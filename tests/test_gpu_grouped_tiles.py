@@ -1,7 +1,7 @@
 """Layers of more than 32 tokens (grouped projections in 16- and 32-route
 m-tiles) against the same tokens in batches of 24, which take the decode
 kernels: bit for bit, at the edges of the tiles, of the tile rules (64, 192,
-512, 576, 1024 and 2048 tokens) and with experts of 1 to several tiles' routes."""
+512, 576, 1024, 2048 and 5120 tokens) and with experts of 1 to several tiles' routes."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,7 @@ from _ornith import Bank, bf16_normal, from_dev, load_shared_tables, moe_weights
 
 pytestmark = pytest.mark.gpu
 DISTINCT = 24
-SIZES = [33, 47, 64, 65, 129, 192, 193, 300, 512, 513, 577, 1024, 1120, 2048, 2049]
+SIZES = [33, 47, 64, 65, 129, 192, 193, 300, 512, 513, 577, 1024, 1120, 2048, 2049, 5120, 5121]
 
 
 def _tokens(rng, T):
