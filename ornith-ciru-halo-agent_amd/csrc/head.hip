@@ -8,6 +8,7 @@
 #include <algorithm>
 #include "kernels.hpp"
 #include "timing.hpp"
+#include "memory_kind.hpp"
 #include "validate.hpp"
 #include "../../include/ornith_head.h"
 
@@ -322,8 +323,9 @@ __global__ __launch_bounds__(64 * kW8Waves, 1) void head_w8_mfma_kernel(
 // blocks meet in argmax[row] itself (cleared by the launch before): one
 // 64-bit atomic maximum per block, and logits_argmax_finish turns the winning
 // key into its column.  W8 head and hand-off at N = 248320, 1 row 341 -> 98 us,
-// 32 rows 400 -> 126 us.  Tokens that live in host memory, where device atomics
-// do not reach, keep one block per row, which walks the parts (11 us alone).
+// 32 rows 400 -> 126 us.  Tokens that live in host memory or on another GPU,
+// where this device's atomics do not reach, keep one block per row, which walks
+// the parts (11 us alone).
 constexpr int kArgThreads = 512, kArgLoads = 4, kArgPart = kArgThreads * 8 * kArgLoads;
 
 __device__ __forceinline__ uint64_t argmax_key(uint32_t b, int c) {
@@ -394,14 +396,14 @@ __global__ __launch_bounds__(64) void logits_argmax_finish_kernel(int M, int64_t
     if (row < M) argmax[row] = int64_t(~uint32_t(uint64_t(argmax[row])));
 }
 
-// Memory of a device (hipMalloc), as opposed to pinned host or managed memory.
-bool device_memory(const void* p) {
+// The device that runs `s` reaches p with device-scope atomics.
+bool atomics_reach(const void* p, hipStream_t s) {
     hipPointerAttribute_t at{};
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
-    return at.type == hipMemoryTypeDevice && !at.isManaged;
+    return device_atomics_reach(at, stream_device(s));
 }
 
 bool head_shape(int N) { return N == 256 || N == 1024 || N == 4096 || N == 65536 || N == 248320; }
@@ -507,7 +509,7 @@ extern "C" hipError_t ornith_logits_argmax_launch(const void* logits_bf16, int M
             timed_launch("logits_argmax", kernel, dim3(parts, std::min(M - r, 65535)), dim3(kArgThreads), 0, stream,
                          src + size_t(r) * size_t(ld), N, ld, dst + r);
     };
-    if (parts == 1 || !device_memory(dst)) {
+    if (parts == 1 || !atomics_reach(dst, stream)) {
         go(logits_argmax_kernel<false>, 1);
         return hipGetLastError();
     }
