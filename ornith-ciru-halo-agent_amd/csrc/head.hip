@@ -314,19 +314,28 @@ __global__ __launch_bounds__(64 * kW8Waves, 1) void head_w8_mfma_kernel(
 // images of the value over the complemented column, so the unsigned maximum is
 // the answer.
 //
-// A row is cut into parts of kArgPart columns, one block each; a thread loads
-// kArgLoads 16-byte pieces before it looks at any of them (a wave reads 1 KB
-// contiguous per load).  Bound by the round trip of those loads: one block per
-// row with 2-byte loads, one at a time, took ~265 us at N = 248320 for 1 row
-// as for 32, three times the head before it; a whole row in one wide block is
-// still ~7 us of key arithmetic on one CU.  With more than one part, the
-// blocks meet in argmax[row] itself (cleared by the launch before): one
-// 64-bit atomic maximum per block, and logits_argmax_finish turns the winning
-// key into its column.  W8 head and hand-off at N = 248320, 1 row 341 -> 98 us,
-// 32 rows 400 -> 126 us.  Tokens that live in host memory or on another GPU,
-// where this device's atomics do not reach, keep one block per row, which walks
-// the parts (11 us alone).
-constexpr int kArgThreads = 512, kArgLoads = 4, kArgPart = kArgThreads * 8 * kArgLoads;
+// A thread loads kArgLoads 16-byte pieces before it looks at any of them (a
+// wave reads 1 KB contiguous per load).  Bound by the round trip of those loads
+// and by the key arithmetic: one block per row with 2-byte loads, one at a
+// time, took ~265 us at N = 248320 for 1 row as for 32, three times the head
+// before it.
+//  - Few long rows are cut into parts of kArgPart columns, one block each, which
+//    meet in argmax[row] itself (cleared by the launch before): one 64-bit
+//    atomic maximum per block, and logits_argmax_finish turns the winning key
+//    into its column.  W8 head and hand-off at N = 248320, 1 row 341 -> 98 us,
+//    32 rows 400 -> 126 us.
+//  - Rows of up to two parts (1 row, N = 16384: 4.0 us walked, 7.3 cut; 32000
+//    5.9 / 7.4; 49000 7.7 / 7.4) and two rows or more per CU (512 rows,
+//    N = 248320: 59 / 63 us, 65536 19.5 / 24.3; 384 rows 57 / 48) keep one block
+//    per row, which walks the parts: one launch in place of three.  So do tokens
+//    in host memory or on another GPU, where this device's atomics do not reach.
+//  - Short rows want fewer threads, whose reduction is then most of the time:
+//    4096 columns and 2048 rows 7.7 us with 512 threads, 5.9 with 256; 1000
+//    columns 6.2 / 4.6, 3.8 with 64 (1 row 2.5 / 2.3; up to 2 columns a thread,
+//    without 16-byte pieces, N = 256 2.5 / 2.0).
+constexpr int kArgThreads = 512, kArgLoads = 4;
+constexpr int kArgPart = kArgThreads * 8 * kArgLoads;
+constexpr int kArgSmallThreads = 256, kArgTinyThreads = 64;
 
 __device__ __forceinline__ uint64_t argmax_key(uint32_t b, int c) {
     const bool nan = (b & 0x7fffu) > 0x7f80u;
@@ -335,42 +344,54 @@ __device__ __forceinline__ uint64_t argmax_key(uint32_t b, int c) {
     return (uint64_t(ord) << 32) | uint32_t(~c);
 }
 
-template <bool SPLIT>
-__global__ __launch_bounds__(kArgThreads) void logits_argmax_kernel(const uint16_t* __restrict__ logits, int N,
-                                                                    int64_t ld, int64_t* __restrict__ argmax) {
-    __shared__ uint64_t s_best[kArgThreads / 64];
+template <bool SPLIT, int THREADS>
+__global__ __launch_bounds__(THREADS) void logits_argmax_kernel(const uint16_t* __restrict__ logits, int N, int64_t ld,
+                                                                int64_t* __restrict__ argmax) {
+    constexpr int kPart = THREADS * kArgLoads;
+    __shared__ uint64_t s_best[THREADS / 64];
     const int row = blockIdx.y, tid = threadIdx.x;
     const uint16_t* src = logits + size_t(row) * size_t(ld);
-    // 16-byte pieces on the address grid: piece p is columns 8 p - lead .. 8 p - lead + 7
-    // (lead columns of the first piece, and those past N, are not the row's)
-    const int lead = int((reinterpret_cast<uintptr_t>(src) >> 1) & 7);
     uint64_t best = 0;
     auto take = [&](uint32_t b, int c) {
         const uint64_t key = argmax_key(b, c);
         best = key > best ? key : best;
     };
-    for (int64_t base = int64_t(blockIdx.x) * kArgPart - lead; base < N; base += int64_t(gridDim.x) * kArgPart) {
-        u32x4 v[kArgLoads];
-        bool whole[kArgLoads];
-#pragma unroll
-        for (int u = 0; u < kArgLoads; ++u) {
-            const int64_t c = base + 8 * (int64_t(u) * kArgThreads + tid);
-            whole[u] = c >= 0 && c + 8 <= N;
-            if (whole[u]) v[u] = *reinterpret_cast<const u32x4*>(src + c);
-        }
-#pragma unroll
-        for (int u = 0; u < kArgLoads; ++u) {
-            const int64_t c = base + 8 * (int64_t(u) * kArgThreads + tid);
-            if (whole[u]) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    take(v[u][e] & 0xffffu, int(c) + 2 * e);
-                    take(v[u][e] >> 16, int(c) + 2 * e + 1);
-                }
-            } else {
-                for (int64_t k = c < 0 ? 0 : c; k < c + 8 && k < N; ++k) take(src[k], int(k));
+    if (THREADS == kArgSmallThreads && N <= 2 * THREADS) {
+        for (int c = tid; c < N; c += THREADS) take(src[c], c);
+    } else {
+        // the row's 16-byte pieces start at its first aligned column; the
+        // up to 7 columns before and after them go to one thread each
+        const int head = min(N, int(-(reinterpret_cast<uintptr_t>(src) >> 1) & 7));
+        const int pieces = (N - head) >> 3;
+        int edge = -1;
+        uint32_t edge_bits = 0;
+        if (blockIdx.x == 0 && tid < 16) {
+            const int c = tid < 8 ? tid : head + 8 * pieces + tid - 8;
+            if (tid < 8 ? c < head : c < N) {
+                edge = c;
+                edge_bits = src[c];
             }
         }
+        for (int p0 = int(blockIdx.x) * kPart; p0 < pieces; p0 += int(gridDim.x) * kPart) {
+            u32x4 v[kArgLoads];
+#pragma unroll
+            for (int u = 0; u < kArgLoads; ++u) {
+                const int p = p0 + u * THREADS + tid;
+                if (p < pieces) v[u] = *reinterpret_cast<const u32x4*>(src + head + 8 * size_t(p));
+            }
+#pragma unroll
+            for (int u = 0; u < kArgLoads; ++u) {
+                const int p = p0 + u * THREADS + tid;
+                if (p < pieces) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        take(v[u][e] & 0xffffu, head + 8 * p + 2 * e);
+                        take(v[u][e] >> 16, head + 8 * p + 2 * e + 1);
+                    }
+                }
+            }
+        }
+        if (edge >= 0) take(edge_bits, edge);
     }
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1) {
@@ -381,9 +402,9 @@ __global__ __launch_bounds__(kArgThreads) void logits_argmax_kernel(const uint16
     __syncthreads();
     if (tid != 0) return;
 #pragma unroll
-    for (int w = 1; w < kArgThreads / 64; ++w) best = s_best[w] > best ? s_best[w] : best;
+    for (int w = 1; w < THREADS / 64; ++w) best = s_best[w] > best ? s_best[w] : best;
     if constexpr (SPLIT) {
-        // (a part past the row's last column, when the lead makes one more, holds no key)
+        // (a part past the row's last piece, where the row starts off the 16-byte grid, holds no key)
         if (best) atomicMax(reinterpret_cast<unsigned long long*>(argmax + row), (unsigned long long)best);
     } else {
         argmax[row] = int64_t(~uint32_t(best));
@@ -499,23 +520,28 @@ extern "C" hipError_t ornith_logits_argmax_launch(const void* logits_bf16, int M
     const Buffer buffers[] = {{logits_bf16, (size_t(M - 1) * size_t(ld) + size_t(N)) * 2, 2, false, false},
                               {argmax_i64, size_t(M) * 8, 8, true, false}};
     if (!check_buffers(buffers)) return hipErrorInvalidValue;
-    // up to 7 columns of lead in the first 16-byte piece
-    const int parts = int((int64_t(N) + 7 + kArgPart - 1) / kArgPart);
+    const int parts = int((int64_t(N) + kArgPart - 1) / kArgPart);
     const auto src = static_cast<const uint16_t*>(logits_bf16);
     const auto dst = static_cast<int64_t*>(argmax_i64);
-    auto go = [&](auto kernel, int parts) {
+    auto go = [&](auto kernel, int parts, int threads) {
         // rows ride on the grid's y axis (65535 blocks at most)
         for (int r = 0; r < M; r += 65535)
-            timed_launch("logits_argmax", kernel, dim3(parts, std::min(M - r, 65535)), dim3(kArgThreads), 0, stream,
+            timed_launch("logits_argmax", kernel, dim3(parts, std::min(M - r, 65535)), dim3(threads), 0, stream,
                          src + size_t(r) * size_t(ld), N, ld, dst + r);
     };
-    if (parts == 1 || !atomics_reach(dst, stream)) {
-        go(logits_argmax_kernel<false>, 1);
+    // (why the lines lie there: logits_argmax_kernel)
+    const bool many = M >= 2 * device_cu_count();
+    if (parts <= 2 || many || !atomics_reach(dst, stream)) {
+        if (many && N > 2 * kArgSmallThreads && N <= 1024)
+            go(logits_argmax_kernel<false, kArgTinyThreads>, 1, kArgTinyThreads);
+        else if (N <= 4096 || (many && N <= 8192))
+            go(logits_argmax_kernel<false, kArgSmallThreads>, 1, kArgSmallThreads);
+        else go(logits_argmax_kernel<false, kArgThreads>, 1, kArgThreads);
         return hipGetLastError();
     }
     hipError_t st = launch_fill_u32(reinterpret_cast<uint32_t*>(dst), size_t(M) * 2, 0u, stream);
     if (st != hipSuccess) return st;
-    go(logits_argmax_kernel<true>, parts);
+    go(logits_argmax_kernel<true, kArgThreads>, parts, kArgThreads);
     st = hipGetLastError();
     if (st != hipSuccess) return st;
     timed_launch("logits_argmax_finish", logits_argmax_finish_kernel, dim3((M + 63) / 64), dim3(64), 0, stream, M, dst);

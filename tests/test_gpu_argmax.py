@@ -1,6 +1,7 @@
 """Greedy hand-off over rows cut into parts: columns on both sides of a part's
-edge, rows that start at every even address, strides other than N, and tokens
-in pinned host memory, against the first-maximum rule."""
+edge, rows that start at every even address, strides other than N, short rows
+and many rows (which one block walks), and tokens in pinned host memory, against
+the first-maximum rule."""
 import numpy as np
 import pytest
 
@@ -14,7 +15,9 @@ PART = 16384                       # columns per block
 
 @pytest.mark.parametrize('M,N,lead', [(1, 1, 0), (2, 7, 3), (3, PART - 7, 7), (3, PART - 6, 7), (3, PART - 6, 1),
                                       (2, PART, 0), (2, PART + 1, 5), (5, 2 * PART + 9, 2), (1, 248320, 0),
-                                      (33, 50001, 4)])
+                                      (33, 50001, 4), (3, 512, 1), (9, 513, 0), (9, 4096, 3), (9, 4097, 1),
+                                      (520, 300, 5), (520, 2049, 6), (513, 2048, 1), (600, 519, 7), (512, 8192, 2),
+                                      (512, 8193, 0), (2, 2 * PART, 1), (2, 2 * PART + 1, 1), (513, 3 * PART + 3, 4), (513, 1024, 1)])
 @pytest.mark.parametrize('host', [False, True])
 def test_argmax_parts(M, N, lead, host):
     import torch
