@@ -73,11 +73,11 @@ hipError_t launch_act_middle(const float* gate_y, int RS, int R, const int32_t* 
                              int32_t* sums, uint32_t* sticky, hipStream_t s);
 
 // ---- routing ---------------------------------------------------------------
-// Wave-per-row router up to here, token-tiled beyond: rows against tiles 10.2 /
-// 13.4 us at 96 tokens, 13.3 / 13.3 at 131, 14.4 / 13.3 at 160, 20.0 / 13.4 at
-// 256 (the tile kernel's blocks are all resident up to 1024 tokens, so its time
-// hardly moves).
-constexpr int kRouterRowsMaxTokens = 144;
+// Wave-per-row router up to here (19 groups of 8 tokens), token-tiled beyond.
+// Router and top-8 as one call, rows / tiles: 144 tokens 16.1 / 17.2 us, 152
+// 17.1 / 17.3, 153 18.3 / 17.3, 200 20.7 / 17.3, 256 24.0 / 17.3 (the tile
+// kernel's blocks are all resident up to 1024 tokens, so its time hardly moves).
+constexpr int kRouterRowsMaxTokens = 152;
 constexpr int kRouterSplitMinTokens = 256;     // the split tail (and its scratch) only beyond
 // Router logits [T, 256 (+1)] in the declared order; shared_w (nullable) adds
 // column 256, the shared-expert gate logit.  split_sums (nullable,

@@ -263,8 +263,8 @@ def test_shared_tables_bit_exact(device, moe, shared_tables, T):
 # ---------------------------------------------------------------------------
 # Router + softmax/top-8 and the whole layer
 # ---------------------------------------------------------------------------
-@pytest.mark.parametrize('T,biased', [(1, False), (33, False), (64, True), (256, False), (257, True), (300, True),
-                                      (700, False)])
+@pytest.mark.parametrize('T,biased', [(1, False), (33, False), (64, True), (152, True), (153, False), (256, False),
+                                      (257, True), (300, True), (700, False)])
 def test_router_topk_bit_exact(device, moe, T, biased):
     import torch
     native = _native()
