@@ -64,31 +64,27 @@ hipError_t run_routed(const RoutedPlan& p, void* ws, const void* input, const fl
                       uint16_t* out, uint16_t* shared_out, uint16_t* layer_out, uint32_t* sticky, int T, int Tcap,
                       hipStream_t s, bool counted = false) {
     const bool shared = sg_codes != nullptr;
-    const int R = T * kTop, RS = R + (shared ? T : 0);
+    const int R = T * kTop;
     const PermuteScratch ps = carve_permute(at<void>(ws, p.permute), Tcap * kTop, shared ? Tcap : 0);
-    // the (otherwise unused) gate_y rows, 4 KiB a route, hold the raw block counts (64 bytes a token, 1 KiB at
-    // least) and the projections' m-tiles
-    int32_t* raw = at<int32_t>(ws, p.l.gate_y);
-    Segment* work = at<Segment>(raw, align256(size_t(T) * 64 + 1024));
-    const int tile_rows = grouped_tile_rows(T);
+    // the m-tiles stand in the (otherwise unused) gate_y rows, 4 KiB a route
+    Segment* tiles = at<Segment>(ws, p.l.gate_y);
+    const int tile_rows = grouped_tile_rows(T), max_tiles = grouped_max_tiles(T, shared);
+    if (size_t(max_tiles) * sizeof(Segment) > p.l.middle - p.l.gate_y) return hipErrorInvalidValue;
     auto gw = at<uint32_t>(ws, p.l.gate_low);
     auto gs = at<uint16_t>(ws, p.l.gate_scales);
     auto gsum = at<int32_t>(ws, p.l.gate_sums);
-    // the A8 gate input rides on the bank-scan launch (the A4 one has its own)
+    // the A8 gate input rides on one of the permutation's launches (the A4 one has its own)
     const ActJob act{static_cast<const uint16_t*>(input), T, shared ? nullptr : ids, gw, gs, gsum};
-    TRY(launch_permute(ids, R, T, shared, ps, sticky, work, tile_rows, raw, s, counted, qmax == 127 ? &act : nullptr));
+    TRY(launch_permute(ids, R, T, shared, ps, sticky, tiles, tile_rows, s, counted, qmax == 127 ? &act : nullptr));
     if (qmax != 127)
         TRY(launch_act_bf16(static_cast<const uint16_t*>(input), kHidden, T, kHidden, qmax, shared ? nullptr : ids, gw,
                             gs, gsum, sticky, kFlagNonfiniteInput, kFlagInvalidActivation, s));
-    const int max_tiles =
-        (RS + tile_rows - 1) / tile_rows + (R < kExperts ? R : kExperts) + (shared ? 1 : 0);
     auto dw = at<uint32_t>(ws, p.l.down_low);
     auto dsc = at<uint16_t>(ws, p.l.down_scales);
     auto dsum = at<int32_t>(ws, p.l.down_sums);
     MfmaArgs a{};
-    a.segments = ps.segments;
-    a.tiles = work;
-    a.ntiles = ps.meta + 2;
+    a.tiles = tiles;
+    a.ntiles = ps.ntiles;
     a.routes = ps.routes;
     a.R = R;
     a.codes = static_cast<const uint32_t*>(gate_codes);
@@ -372,8 +368,7 @@ extern "C" hipError_t ornith_moe_layer_launch(
                       kLogitStride, stream, split));
     TRY(launch_topk(logits, kLogitStride, T, static_cast<float*>(topk_weights), static_cast<int32_t*>(topk_ids),
                     logits + kExperts, kLogitStride, static_cast<uint16_t*>(shared_logit), stream,
-                    permute_fused(T) ? at<int32_t>(workspace, p.l.gate_y) : ps.block_counts,
-                    split, static_cast<const float*>(bias)));
+                    ps.block_counts, split, static_cast<const float*>(bias)));
     return run_routed(p, workspace, input, static_cast<const float*>(topk_weights),
                       static_cast<const int32_t*>(topk_ids), gate_codes, gate_meta, down_codes, down_meta,
                       shared_gate_codes, shared_gate_meta, shared_down_codes, shared_down_meta,
@@ -449,7 +444,7 @@ extern "C" hipError_t ornith_shared_fixed8_launch(const void* input, const void*
 
 // ---- the whole layer without a caller workspace --------------------------------
 // Scratch of ornith_moe_layer_launch_static: the layer plan at Tcap = 32 needs
-// 4,784,896 bytes; 5 MiB per GPU, held for the life of the process.  In host
+// 4,774,656 bytes; 5 MiB per GPU, held for the life of the process.  In host
 // code `scratch` only names the symbol: its device address comes from
 // hipGetSymbolAddress, once per device, and only that address is passed on.
 namespace {

@@ -45,17 +45,14 @@ int resident_blocks(Kernel kernel, int threads, int dev) {
 
 // A run of consecutive entries of the permuted route list that all use one
 // weight bank (expert id 0..255, or kShared for the shared expert).
-struct Segment { int32_t bank, first, count, tile_base; };
+struct Segment { int32_t bank, first, count, index; };
 
 // Scratch used by the permutation step, carved out of the caller's workspace.
 struct PermuteScratch {
-    int32_t* block_counts;   // [blocks, banks]
-    int32_t* counts;         // [banks]
-    int32_t* offsets;        // [banks + 1]
+    int32_t* block_counts;   // [blocks, 256] the blocks' counts, running sums after the bank scan
+    int32_t* counts;         // [256] bank totals (written by the bank scan only)
     int32_t* routes;         // [routes] permuted route ids
-    Segment* segments;       // [banks]
-    int32_t* meta;           // [4]: segment count, 64-route tile count, work tile count
-    Segment* tiles;          // [max tiles] per 64-route tile: bank, first permuted route, rows, tile-in-segment
+    int32_t* ntiles;         // [1] m-tiles
 };
 
 // ---- activations -----------------------------------------------------------
@@ -106,21 +103,19 @@ struct ActJob {
     uint32_t* words; uint16_t* scales; int32_t* sums;
 };
 // Stable counting sort of route ids by bank.  Routes 0..R-1 use ids[r];
-// when with_shared, routes R..R+T-1 use the shared bank.  act (nullable):
-// that quantisation runs as trailing blocks of the bank-scan launch (its 64
-// blocks leave the rest of the chip idle).
-// Up to kPermFusedBlocks 16-token blocks the bank scan is part of the scatter
-// launch (and act's blocks with it): one launch less, every block reading the
-// other blocks' 1 KiB of counts.  The count step then writes to `raw`
-// ([blocks, 256]) instead of block_counts.
+// when with_shared, routes R..R+T-1 use the shared bank.  Up to
+// kPermFusedBlocks 16-token blocks the bank scan is part of the scatter launch:
+// one launch less, every block reading the other blocks' 1 KiB of counts.
+// act (nullable): that quantisation runs as trailing blocks of the scatter
+// launch then, of the bank-scan launch above (whose 64 blocks leave the rest of
+// the chip idle).
+// tiles: the projections' m-tiles of tile_rows routes, per tile {bank, first
+// permuted route, rows, tile in bank}, ascending (counted in ntiles).
 constexpr int kPermFusedBlocks = 128;
-inline bool permute_fused(int T) { return (T + 15) / 16 <= kPermFusedBlocks; }
-// work: the projections' m-tiles of work_rows routes, in the form of
-// PermuteScratch::tiles (counted in meta[2]).
 size_t permute_scratch_bytes(int Rcap, int Tcap);
 PermuteScratch carve_permute(void* base, int Rcap, int Tcap);
 hipError_t launch_permute(const int32_t* ids, int R, int T, bool with_shared, const PermuteScratch& p,
-                          uint32_t* sticky, Segment* work, int work_rows, int32_t* raw, hipStream_t s, bool counted = false,
+                          uint32_t* sticky, Segment* tiles, int tile_rows, hipStream_t s, bool counted = false,
                           const ActJob* act = nullptr);
 
 // ---- projections -----------------------------------------------------------
@@ -156,7 +151,7 @@ hipError_t launch_project_gemv(const ProjArgs& a, int max_segments, Out mode, hi
 
 // Grouped int8-MFMA projection over the permuted routes (prefill path).
 struct MfmaArgs {
-    const Segment* segments; const Segment* tiles; const int32_t* ntiles; const int32_t* routes;
+    const Segment* tiles; const int32_t* ntiles; const int32_t* routes;
     int R;                                       // routed routes; rows >= R are shared-expert rows
     const uint32_t* codes; const uint32_t* meta; const uint32_t* shared_codes; const uint32_t* shared_meta;
     int64_t bank_words, bank_meta_words;
@@ -176,12 +171,17 @@ struct MfmaArgs {
     uint32_t flag_projection, flag_bf16;
 };
 // gate-up (H128 + quantisation of its middle rows included: mid_*) or down of a layer of T > 32 tokens, whose
-// permutation made m-tiles of grouped_tile_rows(T) rows
+// permutation made m-tiles of grouped_tile_rows(T) rows, grouped_max_tiles of them at most
 int grouped_tile_rows(int T);
+inline int grouped_max_tiles(int T, bool shared) {
+    const int R = T * kTop, RS = R + (shared ? T : 0), rows = grouped_tile_rows(T);
+    return (RS + rows - 1) / rows + (R < kExperts ? R : kExperts) + (shared ? 1 : 0);
+}
 hipError_t launch_grouped_mfma(const MfmaArgs& a, bool gateup, int qmax, int T, int max_tiles, hipStream_t s);
 // Dense G256 head on the matrix cores: M <= 64 rows of A8 activations against
 // N32 codes, then the per-row argmax (numpy rule) into argmax[M].
 hipError_t launch_head_mfma(const MfmaArgs& a, int64_t* argmax, hipStream_t s);
+
 // ---- combination -------------------------------------------------------------
 // out[t] = bf16(sum over valid slots of route_out[8t+s] * w[8t+s]); optional
 // fp32 diagnostic; optional shared output and layer sum.

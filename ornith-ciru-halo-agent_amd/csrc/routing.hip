@@ -29,7 +29,6 @@ __device__ __forceinline__ void bf16x8_to_f32(const uint4 v, float f[8]) {
 
 constexpr int kPermTokens = 16;                      // tokens per permutation count / scatter block
 constexpr int kPermRoutes = kPermTokens * kTop;      // routed routes per block
-constexpr int kTileRoutes = 64;                      // routes per m-tile of the scratch's tile list
 
 // ---------------------------------------------------------------------------
 // Router logits for large T on the matrix cores (declared order above).  A
@@ -484,16 +483,7 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) { return wave_prefix_s
 size_t permute_scratch_bytes(int Rcap, int Tcap) {
     const size_t rall = size_t(Rcap) + size_t(Tcap);
     const size_t blocks = (size_t(Rcap / kTop) + kPermTokens - 1) / kPermTokens;
-    size_t bytes = 0;
-    bytes += align256(blocks * kExperts * 4);
-    bytes += align256(kBanks * 4);
-    bytes += align256((kBanks + 1) * 4);
-    bytes += align256(rall * 4);
-    bytes += align256(kBanks * sizeof(Segment));
-    bytes += align256(4 * 4);
-    // one per 64-route m-tile, plus the launch's rounding up to a multiple of 8 tiles
-    bytes += align256((rall / 64 + kBanks + 10) * sizeof(Segment));
-    return bytes;
+    return align256(blocks * kExperts * 4) + align256(kExperts * 4) + align256(rall * 4) + align256(4);
 }
 
 PermuteScratch carve_permute(void* base, int Rcap, int Tcap) {
@@ -503,12 +493,9 @@ PermuteScratch carve_permute(void* base, int Rcap, int Tcap) {
     size_t off = 0;
     auto take = [&](size_t bytes) { void* q = at<void>(base, off); off += align256(bytes); return q; };
     p.block_counts = static_cast<int32_t*>(take(blocks * kExperts * 4));
-    p.counts = static_cast<int32_t*>(take(kBanks * 4));
-    p.offsets = static_cast<int32_t*>(take((kBanks + 1) * 4));
+    p.counts = static_cast<int32_t*>(take(kExperts * 4));
     p.routes = static_cast<int32_t*>(take(rall * 4));
-    p.segments = static_cast<Segment*>(take(kBanks * sizeof(Segment)));
-    p.meta = static_cast<int32_t*>(take(4 * 4));
-    p.tiles = static_cast<Segment*>(take((rall / 64 + kBanks + 10) * sizeof(Segment)));
+    p.ntiles = static_cast<int32_t*>(take(4));
     return p;
 }
 
@@ -519,9 +506,9 @@ PermuteScratch carve_permute(void* base, int Rcap, int Tcap) {
 //   bank scan  one wave per routed bank: exclusive running sums over blocks
 //              (in place) and the bank total; with few blocks each scatter
 //              block forms its own sums instead
-//   scatter    every block scans the 257 bank totals into offsets; block 0
-//              also writes offsets, segments, the MFMA tile list and meta; a
-//              route's slot is offset + running sum + its rank in the block.
+//   scatter    every block scans the 257 bank totals into offsets and writes
+//              its share of the m-tile list (block 0 their number); a route's
+//              slot is offset + running sum + its rank in the block.
 __global__ __launch_bounds__(kPermRoutes) void permute_count_kernel(const int32_t* __restrict__ ids, int T,
                                                                     int32_t* __restrict__ block_counts,
                                                                     uint32_t* sticky) {
@@ -579,22 +566,20 @@ __global__ __launch_bounds__(256) void permute_bank_scan_act_kernel(int nblocks,
                             act.scales, act.sums, sticky, kFlagNonfiniteInput, kFlagInvalidActivation);
 }
 
-// FUSED (at most kPermFusedBlocks blocks): raw holds the blocks' counts as the
-// count step left them; every block sums all of them for itself (its running
-// counts and the totals), and the blocks past nblocks run the activation
+// FUSED (at most kPermFusedBlocks blocks): block_counts holds the blocks' counts
+// as the count step left them; every block sums all of them for itself (its
+// running counts and the totals), and the blocks past nblocks run the activation
 // quantisation (act_bf16_block indices 0, 1, ...).  Otherwise the bank scan has
-// left running counts in block_counts and totals in counts.
+// left running counts there and totals in counts.
 template <bool FUSED>
 __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __restrict__ ids, int T, int shared_routes,
-                                                              int nblocks, const int32_t* __restrict__ raw,
-                                                              int32_t* __restrict__ block_counts,
-                                                              int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
-                                                              int32_t* __restrict__ routes, Segment* __restrict__ segments,
-                                                              int32_t* __restrict__ meta, Segment* __restrict__ tiles,
-                                                              Segment* __restrict__ work, int work_rows, ActJob act,
+                                                              int nblocks, const int32_t* __restrict__ block_counts,
+                                                              const int32_t* __restrict__ counts,
+                                                              int32_t* __restrict__ routes, int32_t* __restrict__ ntiles,
+                                                              Segment* __restrict__ tiles, int tile_rows, ActJob act,
                                                               uint32_t* sticky) {
     __shared__ int s_off[kBanks + 1];        // exclusive route offsets (s_off[257] = live routes)
-    __shared__ int s_tile[2][kBanks + 1];    // exclusive offsets of the 64-route tiles and the work tiles (at 257: all)
+    __shared__ int s_tile[kBanks + 1];       // exclusive m-tile offsets (s_tile[257] = tiles)
     __shared__ __align__(16) int bank_of[kPermRoutes];
     __shared__ __align__(16) int s_total[FUSED ? kExperts : 1];
     __shared__ int s_before[FUSED ? kExperts : 1];
@@ -619,7 +604,7 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
         for (int k0 = 0; k0 < nblocks; k0 += 32) {             // 32 blocks' counts in flight at once
             int v[32];
 #pragma unroll
-            for (int k = 0; k < 32; ++k) v[k] = raw[min(k0 + k, nblocks - 1) * kExperts + tid];
+            for (int k = 0; k < 32; ++k) v[k] = block_counts[min(k0 + k, nblocks - 1) * kExperts + tid];
 #pragma unroll
             for (int k = 0; k < 32; ++k) {
                 total += k0 + k < nblocks ? v[k] : 0;
@@ -628,80 +613,50 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
         }
         s_total[tid] = total;
         s_before[tid] = earlier;
-        block_counts[size_t(blockIdx.x) * kExperts + tid] = earlier;
-        if (blockIdx.x == 0) counts[tid] = total;
         __syncthreads();
     }
     if (tid < 64) {
-        // bank totals -> offsets, non-empty ranks and m-tile offsets (lane holds
-        // banks 4 lane .. 4 lane + 3; the shared bank 256 follows)
-        int tot[4], nt[4], nw[4], ne[4], part = 0, ntp = 0, nwp = 0, nep = 0;
+        // bank totals -> route and m-tile offsets (lane holds banks
+        // 4 lane .. 4 lane + 3; the shared bank 256 follows)
+        int tot[4], nt[4], part = 0, ntp = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             tot[i] = FUSED ? s_total[4 * lane + i] : counts[4 * lane + i];
-            nt[i] = (tot[i] + kTileRoutes - 1) / kTileRoutes;
-            nw[i] = (tot[i] + work_rows - 1) / work_rows;
-            ne[i] = tot[i] > 0 ? 1 : 0;
+            nt[i] = (tot[i] + tile_rows - 1) / tile_rows;
             part += tot[i];
             ntp += nt[i];
-            nwp += nw[i];
-            nep += ne[i];
         }
-        const int incl = wave_inclusive_scan(part), nt_incl = wave_inclusive_scan(ntp);
-        const int nw_incl = wave_inclusive_scan(nwp), ne_incl = wave_inclusive_scan(nep);
-        int off = incl - part, tb = nt_incl - ntp, wb = nw_incl - nwp, seg = ne_incl - nep;
+        int off = wave_inclusive_scan(part) - part, tb = wave_inclusive_scan(ntp) - ntp;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int e = 4 * lane + i;
             s_off[e] = off;
-            s_tile[0][e] = tb;
-            s_tile[1][e] = wb;
-            if (blockIdx.x == 0) {
-                offsets[e] = off;
-                if (tot[i] > 0) segments[seg] = Segment{e, off, tot[i], tb};
-            }
+            s_tile[e] = tb;
             off += tot[i];
             tb += nt[i];
-            wb += nw[i];
-            seg += ne[i];
         }
         if (lane == 63) {
-            const int snt = (shared_routes + kTileRoutes - 1) / kTileRoutes;
-            const int snw = (shared_routes + work_rows - 1) / work_rows;
             s_off[kExperts] = off;
             s_off[kBanks] = off + shared_routes;
-            s_tile[0][kExperts] = tb;
-            s_tile[0][kBanks] = tb + snt;
-            s_tile[1][kExperts] = wb;
-            s_tile[1][kBanks] = wb + snw;
-            if (blockIdx.x == 0) {
-                offsets[kExperts] = off;
-                offsets[kBanks] = off + shared_routes;
-                counts[kExperts] = shared_routes;
-                if (shared_routes > 0) segments[seg] = Segment{kExperts, off, shared_routes, tb};
-                meta[0] = seg + (shared_routes > 0 ? 1 : 0);
-                meta[1] = tb + snt;
-                meta[2] = wb + snw;
-            }
+            s_tile[kExperts] = tb;
+            tb += (shared_routes + tile_rows - 1) / tile_rows;
+            s_tile[kBanks] = tb;
+            if (blockIdx.x == 0) ntiles[0] = tb;
         }
     }
     __syncthreads();
-    // m-tiles of both lists, spread over the grid: tile i belongs to the bank e
-    // with s_tile[e] <= i < s_tile[e + 1] (binary search; empty banks have none)
-    auto list = [&](const int* first_tile, Segment* out, int rows) {
-        const int ntiles = first_tile[kBanks];
-        for (int i = blockIdx.x * 256 + tid; i < ntiles; i += nblocks * 256) {
-            int lo = 0, hi = kBanks;                // first_tile[lo] <= i < first_tile[hi]
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (first_tile[mid] <= i) lo = mid; else hi = mid;
-            }
-            const int k = i - first_tile[lo], total = s_off[lo + 1] - s_off[lo];
-            out[i] = Segment{lo, s_off[lo] + k * rows, min(rows, total - k * rows), k};
+    // m-tiles, spread over the grid: tile i belongs to the bank e with
+    // s_tile[e] <= i < s_tile[e + 1] (binary search; empty banks have none)
+    const int all = s_tile[kBanks];
+    for (int i = blockIdx.x * 256 + tid; i < all; i += nblocks * 256) {
+        int lo = 0, hi = kBanks;                    // s_tile[lo] <= i < s_tile[hi]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (s_tile[mid] <= i) lo = mid; else hi = mid;
         }
-    };
-    list(s_tile[0], tiles, kTileRoutes);
-    list(s_tile[1], work, work_rows);
+        const int k = i - s_tile[lo], total = s_off[lo + 1] - s_off[lo];
+        tiles[i] = Segment{lo, s_off[lo] + k * tile_rows, min(tile_rows, total - k * tile_rows), k};
+    }
     if (FUSED && b >= 0) before = s_before[b];
     if (tid < kPermRoutes && b >= 0) {
         // rank in the block = earlier routes of the block with bank b: all of
@@ -726,27 +681,23 @@ __global__ __launch_bounds__(256) void permute_scatter_kernel(const int32_t* __r
 }
 
 hipError_t launch_permute(const int32_t* ids, int R, int T, bool with_shared, const PermuteScratch& p,
-                          uint32_t* sticky, Segment* work, int work_rows, int32_t* raw, hipStream_t s, bool counted,
-                          const ActJob* act) {
+                          uint32_t* sticky, Segment* tiles, int tile_rows, hipStream_t s, bool counted, const ActJob* act) {
     if (R != T * kTop) return hipErrorInvalidValue;
     const int nblocks = (T + kPermTokens - 1) / kPermTokens;
     if (nblocks > 8 * 64) return hipErrorInvalidValue;
-    const bool fused = nblocks <= kPermFusedBlocks;
-    if (fused && !raw) return hipErrorInvalidValue;
-    int32_t* step1 = fused ? raw : p.block_counts;
     if (!counted) {
-        timed_launch("permute_count", permute_count_kernel, dim3(nblocks), dim3(kPermRoutes), 0, s, ids, T, step1,
-                     sticky);
+        timed_launch("permute_count", permute_count_kernel, dim3(nblocks), dim3(kPermRoutes), 0, s, ids, T,
+                     p.block_counts, sticky);
         const hipError_t st = hipGetLastError();
         if (st != hipSuccess) return st;
     }
     // act_bf16_block: four 4-group waves per block index
     const int act_blocks = act ? (act->rows * (kHidden / kGroup) + 15) / 16 : 0;
     const ActJob job = act ? *act : ActJob{};
-    if (fused) {
+    if (nblocks <= kPermFusedBlocks) {
         timed_launch("permute_scatter_act", permute_scatter_kernel<true>, dim3(nblocks + act_blocks), dim3(256), 0, s,
-                     ids, T, with_shared ? T : 0, nblocks, raw, p.block_counts, p.counts, p.offsets, p.routes,
-                     p.segments, p.meta, p.tiles, work, work_rows, job, sticky);
+                     ids, T, with_shared ? T : 0, nblocks, p.block_counts, p.counts, p.routes, p.ntiles, tiles,
+                     tile_rows, job, sticky);
         return hipGetLastError();
     }
     if (act)
@@ -758,8 +709,8 @@ hipError_t launch_permute(const int32_t* ids, int R, int T, bool with_shared, co
     hipError_t st = hipGetLastError();
     if (st != hipSuccess) return st;
     timed_launch("permute_scatter", permute_scatter_kernel<false>, dim3(nblocks), dim3(256), 0, s, ids, T,
-                 with_shared ? T : 0, nblocks, static_cast<const int32_t*>(nullptr), p.block_counts, p.counts,
-                 p.offsets, p.routes, p.segments, p.meta, p.tiles, work, work_rows, job, sticky);
+                 with_shared ? T : 0, nblocks, p.block_counts, p.counts, p.routes, p.ntiles, tiles, tile_rows, job,
+                 sticky);
     return hipGetLastError();
 }
 
