@@ -78,10 +78,11 @@ def kernel_cost(name, T, unique):
     if name in ('down1', 'down'):
         return 'hbm', banks * DOWN_BYTES + routes * 512 * 4 + T * 2048 * 2, HBM_PEAK_GBS, 'GB/s'
     if name in ('gateup_mfma', 'down_mfma'):
-        if name == 'gateup_mfma':       # codes + meta, A8 gate input in, middle rows out (priced as fp32)
-            nbytes, ops = banks * GATEUP_BYTES + T * 2048 + routes * 512 * 4, 2 * routes * 1024 * 2048
+        middle = routes * (512 + 2 * (2 + 4))   # A8 middle rows: codes, and per group an fp16 scale and an int32 sum
+        if name == 'gateup_mfma':       # codes + meta, A8 gate input in, A8 middle rows out
+            nbytes, ops = banks * GATEUP_BYTES + T * 2048 + middle, 2 * routes * 1024 * 2048
         else:                           # codes + meta, A8 middle rows in, fp32 route rows out
-            nbytes, ops = banks * DOWN_BYTES + routes * 512 + routes * 2048 * 4, 2 * routes * 2048 * 512
+            nbytes, ops = banks * DOWN_BYTES + middle + routes * 2048 * 4, 2 * routes * 2048 * 512
         if nbytes / (HBM_PEAK_GBS * 1e9) >= ops / (INT8_PEAK_TOPS * 1e12):
             return 'hbm', nbytes, HBM_PEAK_GBS, 'GB/s'
         return 'mfma', ops, INT8_PEAK_TOPS, 'TFLOP/s'
