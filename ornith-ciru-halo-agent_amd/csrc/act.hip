@@ -2,8 +2,6 @@
 // quantisation into the int8 layout described in common.hpp.
 //   act_bf16   - routed gate / dense input (routed_storage_n32_consumer.cpp:22-76,
 //                dense_g256_consumer.cpp:27-73, dense_n32 :276-322)
-//   act_middle - SiLU(gate)*up, then transform + quantise of the down input
-//                (routed_storage_n32_consumer.cpp:168-175, 231-295)
 // One wave owns one (row, 256-group); four waves per block.
 #include "kernels.hpp"
 #include "timing.hpp"
@@ -21,50 +19,6 @@ __global__ __launch_bounds__(256) void act_bf16_kernel(const uint16_t* __restric
                          flag_act);
 }
 
-template <int QMAX>
-__global__ __launch_bounds__(256) void act_middle_kernel(const float* __restrict__ gate_y, int RS, int R,
-                                                         const int32_t* __restrict__ ids,
-                                                         const float* __restrict__ silu_table,
-                                                         uint32_t* __restrict__ words, uint16_t* __restrict__ scales,
-                                                         int32_t* __restrict__ sums, uint32_t* sticky) {
-    constexpr int groups = kInter / kGroup;
-    const int wave = (blockIdx.x * 4) + (threadIdx.x >> 6);
-    if (wave >= RS * groups) return;
-    const int lane = threadIdx.x & 63;
-    const int route = wave / groups, group = wave % groups;
-    uint32_t flags = 0;
-    const bool shared = route >= R;
-    float v[4];
-    if (!shared && (ids[route] < 0 || ids[route] >= kExperts)) {
-        v[0] = v[1] = v[2] = v[3] = 0.f;
-    } else {
-        const float4 g = *reinterpret_cast<const float4*>(gate_y + size_t(route) * (2 * kInter) + group * kGroup + lane * 4);
-        const float4 u = *reinterpret_cast<const float4*>(gate_y + size_t(route) * (2 * kInter) + kInter + group * kGroup + lane * 4);
-        const float gg[4] = {g.x, g.y, g.z, g.w}, uu[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float value;
-            if (shared) {
-                // Shared rows: tabulated SiLU of the bf16 gate value, product
-                // rounded to bf16 (routed_storage_n32_consumer.cpp:246-250).
-                const float silu = silu_table[__float_as_uint(gg[i]) >> 16];
-                value = bf16_round(silu * uu[i]);
-            } else {
-                const float silu = silu_portable(gg[i]);
-                value = silu * uu[i];
-            }
-            if (!isfinite(value)) flags |= kFlagNonfiniteMiddle | kFlagNonfiniteInput;
-            v[i] = value;
-        }
-    }
-    h128_wave(v);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) if (!isfinite(v[i])) flags |= kFlagNonfiniteInput;
-    quantize_group_wave<QMAX>(v, words + (size_t(route) * groups + group) * 64, scales + size_t(route) * groups + group,
-                              sums + size_t(route) * groups + group, flags, kFlagInvalidActivation);
-    flag_or(sticky, flags);
-}
-
 hipError_t launch_act_bf16(const uint16_t* x, int64_t stride, int rows, int K, int qmax, const int32_t* ids,
                            uint32_t* words, uint16_t* scales, int32_t* sums, uint32_t* sticky,
                            uint32_t flag_input, uint32_t flag_act, hipStream_t s) {
@@ -80,43 +34,7 @@ hipError_t launch_act_bf16(const uint16_t* x, int64_t stride, int rows, int K, i
     return hipGetLastError();
 }
 
-hipError_t launch_act_middle(const float* gate_y, int RS, int R, const int32_t* ids, int qmax,
-                             const float* silu_table, uint32_t* words, uint16_t* scales, int32_t* sums,
-                             uint32_t* sticky, hipStream_t s) {
-    const int waves = RS * (kInter / kGroup);
-    const dim3 grid((waves + 3) / 4), block(256);
-    if (qmax == 127)
-        timed_launch("act_middle", act_middle_kernel<127>, dim3(grid), dim3(block), 0, s, gate_y, RS, R, ids, silu_table, words, scales, sums, sticky);
-    else
-        timed_launch("act_middle", act_middle_kernel<7>, dim3(grid), dim3(block), 0, s, gate_y, RS, R, ids, silu_table, words, scales, sums, sticky);
-    return hipGetLastError();
-}
-
 // ---- dense bf16 prefill operands (dense_g256_consumer.cpp:192-229) ----------
-__global__ __launch_bounds__(256) void transform_bf16_kernel(const uint16_t* __restrict__ x, int M, int groups,
-                                                             uint16_t* __restrict__ y, uint32_t* sticky) {
-    const int wave = (blockIdx.x * 4) + (threadIdx.x >> 6);
-    if (wave >= M * groups) return;
-    const int lane = threadIdx.x & 63;
-    const size_t base = size_t(wave) * kGroup + lane * 4;
-    uint32_t flags = 0;
-    const uint2 raw = *reinterpret_cast<const uint2*>(x + base);
-    float v[4] = {bf16_bits_to_f32(raw.x & 0xffffu), bf16_bits_to_f32(raw.x >> 16),
-                  bf16_bits_to_f32(raw.y & 0xffffu), bf16_bits_to_f32(raw.y >> 16)};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) if (!isfinite(v[i])) flags |= kDenseNonfiniteInput;
-    h128_wave(v);
-    uint16_t r[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if (!isfinite(v[i])) flags |= kDenseNonfiniteInput;
-        r[i] = f32_to_bf16_bits(v[i]);
-        if ((r[i] & 0x7f80u) == 0x7f80u) flags |= kDenseNonfiniteBf16;
-    }
-    *reinterpret_cast<uint2*>(y + base) = make_uint2(r[0] | (uint32_t(r[1]) << 16), r[2] | (uint32_t(r[3]) << 16));
-    flag_or(sticky, flags);
-}
-
 // Four packed code words per thread (32 bf16 weights RN(RN(s*code)+off)).
 // Threads walk the code words in storage order ([N/tile, K/256, 32, tile]:
 // column fastest), four adjacent columns each, so a wave reads one contiguous
@@ -157,12 +75,6 @@ __global__ __launch_bounds__(256) void dequantize_bf16_kernel(const uint32_t* __
         *reinterpret_cast<uint4*>(w + size_t(n) * K + size_t(kw) * 8) = make_uint4(out[0], out[1], out[2], out[3]);
     }
     flag_or(sticky, flags);
-}
-
-hipError_t launch_transform_bf16(const uint16_t* x, int M, int K, uint16_t* y, uint32_t* sticky, hipStream_t s) {
-    const int waves = M * (K / kGroup);
-    timed_launch("transform", transform_bf16_kernel, dim3((waves + 3) / 4), dim3(256), 0, s, x, M, K / kGroup, y, sticky);
-    return hipGetLastError();
 }
 
 hipError_t launch_dequantize_bf16(const uint32_t* codes, const uint32_t* meta, int N, int K, int tile, uint16_t* w,

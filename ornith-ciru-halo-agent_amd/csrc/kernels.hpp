@@ -62,13 +62,6 @@ struct PermuteScratch {
 hipError_t launch_act_bf16(const uint16_t* x, int64_t stride, int rows, int K, int qmax,
                            const int32_t* ids, uint32_t* words, uint16_t* scales, int32_t* sums,
                            uint32_t* sticky, uint32_t flag_input, uint32_t flag_act, hipStream_t s);
-// Middle (SiLU(gate) * up) + H128 + quantisation for RS route rows of
-// gate_y [RS, 1024].  Rows >= R are shared-expert rows (table SiLU, bf16
-// rounding) when silu_table != nullptr.
-hipError_t launch_act_middle(const float* gate_y, int RS, int R, const int32_t* ids, int qmax,
-                             const float* silu_table, uint32_t* words, uint16_t* scales,
-                             int32_t* sums, uint32_t* sticky, hipStream_t s);
-
 // ---- routing ---------------------------------------------------------------
 // Wave-per-row router up to here (19 groups of 8 tokens), token-tiled beyond.
 // Router and top-8 as one call, rows / tiles: 144 tokens 16.1 / 17.2 us, 152
@@ -191,7 +184,6 @@ hipError_t launch_reduce(const float* route_out, const float* weights, const int
                          uint32_t* sticky, hipStream_t s);
 
 // ---- dense bf16 preparation (dense_g256_consumer.cpp:192-246) ---------------
-hipError_t launch_transform_bf16(const uint16_t* x, int M, int K, uint16_t* y, uint32_t* sticky, hipStream_t s);
 hipError_t launch_dequantize_bf16(const uint32_t* codes, const uint32_t* meta, int N, int K, int tile,
                                   uint16_t* w, uint32_t* sticky, hipStream_t s);
 
