@@ -14,11 +14,21 @@
  * ornith_mi355x_timing_names(out, capacity): comma-separated distinct names
  *   recorded so far; returns the length of the full list.
  *
- * Kernel names: route1, gateup1, down1 (single token); route, gateup, down
- * (2..32 tokens); router, topk, permute_count, permute_scan,
- * permute_scatter, act, gateup_mfma, quant_middle, down_mfma, reduce
- * (prefill); dense_gemv, head_encode, head_project, argmax, act_middle,
- * transform, dequantize, fill. */
+ * Kernel names:
+ *   single token     layer1 (one launch); route1, gateup1, down1 (three)
+ *   2..32 tokens     route_select, or route and sort; gateup, down
+ *   prefill          router, topk, permute_count (routed entries),
+ *                    permute_scatter_act (up to 2048 tokens: bank scan, scatter
+ *                    and the 8-bit gate-input quantisation), permute_scan or
+ *                    permute_scan_act and permute_scatter (more), act (4-bit
+ *                    gate input), gateup_mfma (which quantises its middle rows
+ *                    itself), down_mfma, reduce
+ *   dense            act, dense_stream, dense_gemv, dense_gemm, dense_slices,
+ *                    transform_bf16, transform_bf16_frag, dequantize
+ *   heads            head_encode, head_w8_mfma, act, head_mfma, argmax,
+ *                    logits_argmax, logits_argmax_finish (long rows), fill
+ *   shared expert    fixed8_act, fixed8_gate
+ *   other            repack_codes, repack_meta, silu_selfcheck */
 #ifndef ORNITH_TIMING_H
 #define ORNITH_TIMING_H
 #include <hip/hip_runtime_api.h>

@@ -41,6 +41,18 @@ def test_every_declared_symbol_is_exported(tile):
         assert exported == names
 
 
+def test_timing_header_names_every_kernel():
+    text = (ROOT / 'include' / 'ornith_timing.h').read_text()
+    listed = text[text.index('Kernel names:'):text.index('*/')]
+    csrc = ROOT / 'ornith-ciru-halo-agent_amd' / 'csrc'
+    launched = {n for f in sorted(csrc.glob('*.h*')) for n in re.findall(r'timed_launch\(\s*"(\w+)"', f.read_text())}
+    assert len(launched) > 30
+    words = set(re.findall(r'\w+', listed))
+    assert launched <= words, launched - words
+    # and no name of a launch that is gone
+    assert {w for w in words if '_' in w} <= launched
+
+
 def test_markers(lib):
     from ornith_g256 import native
     assert lib.ornith_routed_storage_n32() == 32
