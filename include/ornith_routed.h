@@ -24,7 +24,13 @@
  * Contract differences (all stricter, none in arithmetic):
  *   - workspace internals are this library's own; OrnithRoutedDirectLayout keeps
  *     the reference field names and order but fields this library does not use
- *     have size zero, so workspace_bytes differs from the reference's;
+ *     have size zero, so workspace_bytes differs from the reference's.  Only
+ *     final_f32 (routed entries: the fp32 rows before the bf16 rounding) and
+ *     route_out (2 tokens or more: the fp32 route rows) hold a result after a
+ *     call.  middle holds the fp32 middle rows of 2..32 tokens; above 32 it is
+ *     not written: the gate-up projection hands quantised rows on in down_low,
+ *     down_scales and down_sums (in expert order), and gate_y then holds the
+ *     projections' tile list;
  *   - alignment: input 16 bytes, codes 16 bytes, workspace 256 bytes;
  *   - Tcap <= 8192 for every entry (the reference's N16 parent allowed 2048).
  * Sticky flags (uint32, OR-ed, never cleared): 1 non-finite input/transform,
