@@ -460,15 +460,21 @@ hipError_t launch_tiles(const MfmaArgs& a, bool gateup, int qmax, int max_tiles,
 
 // Rows per m-tile.  Few routes per expert: 16-row tiles, whose kernels keep
 // four waves per SIMD streaming codes; with more routes 32-row tiles read the
-// codes and unpack them half as often (two waves per SIMD).  Layer time, 16
-// against 32 rows: N32 banks 135 / 147 us at 256 tokens, 148 / 153 at 512,
-// 171 / 158 at 700 (even routing), 149 / 143 at 1120 (Zipf 1.1); N16 banks
-// (routed projections alone) 103 / 106 at 80, 130 / 128 at 400, 139 / 135 at
-// 550.  With N16 banks 16-row tiles come back where an even share (T / 32
-// routes) comes close to 32: a few experts beyond it put the 32-row blocks just
-// past one round of the chip's 512 slots (even routing 144 / 159 at 700, 153 /
-// 163 at 900; Zipf 1.2 91 / 86 at 700), until two tiles an expert are the rule
-// (167 / 164 at 1100).
+// codes and unpack them half as often.  Between 200 and 1100 tokens the better
+// height follows the number of 32-row gate-up blocks against the chip's 512
+// slots, which hangs on the routing: spread evenly over the experts it ends up
+// just past a round of them, skewed well below.  T is all the host knows, so
+// each line lies where neither kind of routing loses much.  Per call in us, 16 /
+// 32 rows, even routing and Zipf 1.1 (1.4 at 720):
+//                  320            480            560            720            1024           1200
+//   N32, layer     126/135 82/86  127/146 95/95  137/150 101/101 145/155 110/101 162/163 137/134 183/175 157/154
+//   N32, routed    114/108 63/65  112/115 77/73  122/124 82/79  124/142 87/81  138/145 111/113 151/153 125/123
+//   N16, layer     131/138 83/87  132/148 96/95  141/152 102/101 149/159 111/101 165/166 139/134 186/178 159/156
+//   N16, routed    119/111 64/65  117/118 79/74  127/128 82/80  129/145 88/80  143/148 112/112 155/155 127/123
+// The 64-row tiles before these took, for the routed entries, 115 / 73 us at 320,
+// 139 / 93 (N32) and 135 / 93 (N16) at 720 and 167 / 139 at 1200: 16 rows on
+// N16 banks at 320 and 32 rows there at 720 would be slower than that on evenly
+// routed batches.  N32 routed projections alone at 640-720 tokens are, by 1-2 %.
 int grouped_tile_rows(int T) {
     if (kRoutedTile == 32) return T <= 512 ? 16 : 32;
     return T <= 192 || (T > 576 && T <= 1024) ? 16 : 32;
