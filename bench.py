@@ -51,11 +51,11 @@ DENSE_N = 6144
 MEASURED_TRAFFIC = {
     ('layer1', 1): 16768264, ('route1', 1): 1166652, ('gateup1', 1): 9949504, ('down1', 1): 5118494,
     ('route_select', 32): 5329307, ('gateup', 32): 176476340, ('down', 32): 94490777, ('reduce', 32): 2596402,
-    ('router', 1120): 15343159, ('topk', 1120): 2186694, ('permute_scatter_act', 1120): 7971476,
-    ('gateup_mfma', 1120): 137523438, ('down_mfma', 1120): 146047665, ('reduce', 1120): 87588630,
-    ('router', 8192): 50519792, ('topk', 8192): 9599227, ('permute_scan_act', 8192): 56091210,
-    ('permute_scatter', 8192): 1569102, ('gateup_mfma', 8192): 320505027, ('down_mfma', 8192): 709583375,
-    ('reduce', 8192): 639837397,
+    ('router', 1120): 15327727, ('topk', 1120): 2207752, ('permute_scatter_act', 1120): 7863880,
+    ('gateup_mfma', 1120): 137435948, ('down_mfma', 1120): 144337068, ('reduce', 1120): 87588550,
+    ('router', 8192): 50504386, ('topk', 8192): 9609385, ('permute_scan_act', 8192): 56094414,
+    ('permute_scatter', 8192): 1545844, ('gateup_mfma', 8192): 320702722, ('down_mfma', 8192): 708114258,
+    ('reduce', 8192): 639837375,
 }
 
 
