@@ -366,10 +366,10 @@ __global__ __launch_bounds__(THREADS) void logits_argmax_kernel(const uint16_t* 
         int edge = -1;
         uint32_t edge_bits = 0;
         if (blockIdx.x == 0 && tid < 16) {
-            const int c = tid < 8 ? tid : head + 8 * pieces + tid - 8;
-            if (tid < 8 ? c < head : c < N) {
-                edge = c;
-                edge_bits = src[c];
+            const int left = N - head - 8 * pieces;            // columns after the last piece
+            if (tid < 8 ? tid < head : tid - 8 < left) {
+                edge = tid < 8 ? tid : N - left + tid - 8;
+                edge_bits = src[edge];
             }
         }
         for (int p0 = int(blockIdx.x) * kPart; p0 < pieces; p0 += int(gridDim.x) * kPart) {
