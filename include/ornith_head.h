@@ -56,7 +56,9 @@ ORNITH_EXPORT hipError_t ornith_head_i8_tile_launch(
  * the column of row m's maximum bf16 logit (the first NaN if the row has
  * one, else the first maximum, as torch.argmax / numpy.argmax).  logits
  * bf16 [M, N] with row stride ld >= N elements; M == 0 or N == 0 returns
- * hipSuccess without touching memory. */
+ * hipSuccess without touching memory.  argmax_i64 may be memory of the stream's
+ * device, of a peer or of the host (pinned or managed); its words hold no
+ * columns before the launch has finished. */
 ORNITH_EXPORT hipError_t ornith_logits_argmax_launch(const void* logits_bf16, int M, int N, int64_t ld,
                                                      void* argmax_i64, hipStream_t stream);
 
